@@ -33,9 +33,12 @@ struct rvk_volume {
   uint8_t* gradmag[RVK_MAX_FRAMES] = {};  // u8 cell volumes
   float gradmag_scale[RVK_MAX_FRAMES] = {};
   // Value range (min, max) of every brick of kRangeEdge^3 cells, for the DRR
-  // march's empty-space skipping; nrb = ceil((dims + 2) / kRangeEdge).
+  // march's empty-space skipping; nrb = ceil((dims + 2) / kRangeEdge).  The
+  // allocation ends with the totals an upload collects (frame_stats).
   float2* ranges[RVK_MAX_FRAMES] = {};
   int nrb[3] = {0, 0, 0};
+  size_t n_range_bricks() const { return (size_t)nrb[0] * nrb[1] * nrb[2]; }
+  int* frame_stats(int f) const { return reinterpret_cast<int*>(ranges[f] + n_range_bricks()); }
   // bumped whenever the frames' cells move (rvk_volume_relayout): graphs
   // captured before hold stale cell pointers and are not replayed
   unsigned generation = 0;

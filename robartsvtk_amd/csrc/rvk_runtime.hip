@@ -262,34 +262,116 @@ static int launch_relayout(rvk_volume* v, const void* dsrc, void* dst) {
   return RVK_OK;
 }
 
-// (min, max) of the voxels each range brick's cells reach.  The y and z
+// Value statistics of a frame in one pass over its native voxels.
+//
+// Ranges: (min, max) of the voxels each range brick's cells reach, i.e.
+// voxels [8b - 1, 8b + 7] per axis, clamped into the volume.  The y and z
 // lerps round the difference of their operands, so an interpolated value may
 // leave the voxels' range by a few ulp of the largest magnitude: the bounds
 // of a non-constant brick are widened by 2^-20 of it.  A constant brick
 // interpolates its value exactly and keeps min == max.  A brick with a
 // non-finite voxel gets (-inf, +inf): no run is ever taken through it.
+//
+// Encoding (16-bit frames, stats != NULL): the frame's value range and
+// whether some x-neighbour difference is not exact in binary16 (|d| > 2048
+// and odd; used only for frames within [-2048, 2048], whose differences are
+// at most 4096) decide the cell encoding.
+//
+// One wave per 8 bricks of a brick row: lane l takes column x = 64 c + l
+// through the bricks' 81 voxel rows and reads it with its left neighbour, so
+// an aligned group of 8 lanes covers a brick's 9 columns; the loads of a row
+// are one or two lines, 9 rows in flight (loaded into registers before any is
+// used; with the compares between the loads 256^3 f32 took 79 us).  Bound by
+// that load chain: 250 x 250 x 181 int16 11.9 us, 256^3 f32 21 us (3.2 TB/s).
+// One thread per brick, reading 729 strided voxels, took 79 and 128 us, and
+// the int16 totals, every wave's min and max on one pair of addresses
+// (16384 waves), 380 us more.  The totals go to kStatSlots slots on lines of
+// their own, the blocks dealt over them.
+constexpr int kStatSlots = 64;
+constexpr int kStatStride = 16;  // ints: a 64-byte line per slot
+constexpr size_t kStatBytes = sizeof(int) * kStatSlots * kStatStride;
+
+__global__ __launch_bounds__(kStatSlots) void stats_init_kernel(int* stats) {
+  int* s = stats + threadIdx.x * kStatStride;
+  s[0] = 0x7fffffff;
+  s[1] = -0x7fffffff - 1;
+  s[2] = 0;
+}
+
 template <typename VT>
-__global__ __launch_bounds__(256) void brick_range_kernel(const VT* __restrict__ src, int nx, int ny, int nz, int rbx,
-                                                          int rby, int rbz, float2* __restrict__ out) {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= rbx * rby * rbz) return;
-  const int bx = b % rbx, by = (b / rbx) % rby, bz = b / (rbx * rby);
-  const int x0 = max(bx * kRangeEdge - 1, 0), x1 = min(bx * kRangeEdge + kRangeEdge - 1, nx - 1);
-  const int y0 = max(by * kRangeEdge - 1, 0), y1 = min(by * kRangeEdge + kRangeEdge - 1, ny - 1);
-  const int z0 = max(bz * kRangeEdge - 1, 0), z1 = min(bz * kRangeEdge + kRangeEdge - 1, nz - 1);
+__global__ __launch_bounds__(256) void frame_stats_kernel(const VT* __restrict__ src, int nx, int ny, int nz, int rbx,
+                                                          int rby, int rbz, float2* __restrict__ out, int* stats) {
+  constexpr bool kInt16 = sizeof(VT) == 2;
+  const int lane = threadIdx.x & 63;
+  const int chunks = (rbx + 7) / 8;
+  const int task = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float inf = __builtin_huge_valf();
   float lo = inf, hi = -inf;
-  bool finite = true;
-  for (int k = z0; k <= z1; ++k)
-    for (int j = y0; j <= y1; ++j)
-      for (int i = x0; i <= x1; ++i) {
-        const float v = (float)src[(long long)i + (long long)j * nx + (long long)k * nx * ny];
-        finite = finite && isfinite(v);
-        lo = fminf(lo, v);
-        hi = fmaxf(hi, v);
+  int finite = 1;
+  int odd = 0;
+  const bool has_task = task < chunks * rby * rbz;
+  if (has_task) {
+    const int c = task % chunks, by = (task / chunks) % rby, bz = task / (chunks * rby);
+    const int col = c * 64 + lane;
+    const int x = min(col, nx - 1), xl = min(max(col - 1, 0), nx - 1);
+    for (int k = 0; k < 9; ++k) {
+      const int z = min(max(bz * kRangeEdge - 1 + k, 0), nz - 1);
+      const VT* slab = src + (size_t)z * ny * nx;
+      VT rv[9], rl[9];  // the 9 rows' loads are issued together
+#pragma unroll
+      for (int j = 0; j < 9; ++j) {
+        const VT* row = slab + (size_t)min(max(by * kRangeEdge - 1 + j, 0), ny - 1) * nx;
+        rv[j] = row[x];
+        rl[j] = row[xl];
       }
-  const float w = hi > lo ? fmaxf(fabsf(lo), fabsf(hi)) * 0x1p-20f : 0.0f;
-  out[b] = finite ? make_float2(lo - w, hi + w) : make_float2(-inf, inf);
+#pragma unroll
+      for (int j = 0; j < 9; ++j) {
+        const float v = (float)rv[j], l = (float)rl[j];
+        if constexpr (std::is_same<VT, float>::value) finite = finite & (int)isfinite(v) & (int)isfinite(l);
+        lo = fminf(lo, fminf(v, l));
+        hi = fmaxf(hi, fmaxf(v, l));
+        if constexpr (kInt16) {
+          const int d = abs((int)rv[j] - (int)rl[j]);
+          odd |= (int)(d > 2048 && (d & 1));
+        }
+      }
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      lo = fminf(lo, __shfl_xor(lo, o, 64));
+      hi = fmaxf(hi, __shfl_xor(hi, o, 64));
+    }
+    const unsigned long long bad = __ballot(!finite);
+    const int bx = c * 8 + (lane >> 3);
+    if ((lane & 7) == 0 && bx < rbx) {
+      const float w = hi > lo ? fmaxf(fabsf(lo), fabsf(hi)) * 0x1p-20f : 0.0f;
+      const bool ok = ((bad >> lane) & 0xffull) == 0ull;
+      out[((size_t)bz * rby + by) * rbx + bx] = ok ? make_float2(lo - w, hi + w) : make_float2(-inf, inf);
+    }
+  }
+  if constexpr (kInt16) {
+    // every voxel is in some brick: the bricks' extremes are the frame's
+    __shared__ int s_lo[4], s_hi[4], s_odd[4];
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) {
+      lo = fminf(lo, __shfl_xor(lo, o, 64));
+      hi = fmaxf(hi, __shfl_xor(hi, o, 64));
+    }
+    const bool any_odd = __ballot(odd) != 0ull;
+    if (lane == 0) {
+      const int w = threadIdx.x >> 6;
+      s_lo[w] = has_task ? (int)lo : 0x7fffffff;
+      s_hi[w] = has_task ? (int)hi : -0x7fffffff - 1;
+      s_odd[w] = any_odd;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int* s = stats + (blockIdx.x % kStatSlots) * kStatStride;
+      atomicMin(s, min(min(s_lo[0], s_lo[1]), min(s_lo[2], s_lo[3])));
+      atomicMax(s + 1, max(max(s_hi[0], s_hi[1]), max(s_hi[2], s_hi[3])));
+      if (s_odd[0] | s_odd[1] | s_odd[2] | s_odd[3]) atomicMax(s + 2, 1);
+    }
+  }
 }
 
 // Binary16 cells -> difference cells: each x-pair's base (and, for
@@ -316,59 +398,49 @@ int frame_drop_half(const rvk_volume* cv, int frame, hipStream_t s) {
   return RVK_OK;
 }
 
-// Value range of a 16-bit frame and whether some x-neighbour difference is
-// not exact in binary16 (|d| > 2048 and odd; the flag is used only for
-// frames within [-2048, 2048], whose differences are at most 4096): these
-// decide the frame's cell encoding.
-__global__ __launch_bounds__(64) void range_init_kernel(int* out) {
-  if (threadIdx.x == 0) {
-    out[0] = 0x7fffffff;
-    out[1] = -0x7fffffff - 1;
-    out[2] = 0;
-  }
-}
+// The frame's range bricks from its native voxels on the device, and for
+// 16-bit frames its value range and odd-difference flag (waits for them).
+// The slots of the totals follow the frame's ranges in one allocation.
 template <typename VT>
-__global__ __launch_bounds__(256) void range_kernel(const VT* __restrict__ src, long long n, int nx, int* out) {
-  int lo = 0x7fffffff, hi = -0x7fffffff - 1, odd = 0;
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-    const int x = (int)src[i];
-    lo = min(lo, x);
-    hi = max(hi, x);
-    if ((int)(i % nx) != nx - 1) {
-      const int d = abs((int)src[i + 1] - x);
-      odd |= (int)(d > 2048 && (d & 1));
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = min(lo, __shfl_xor(lo, o, 64));
-    hi = max(hi, __shfl_xor(hi, o, 64));
-    odd |= __shfl_xor(odd, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicMin(out, lo);
-    atomicMax(out + 1, hi);
-    if (odd) atomicMax(out + 2, 1);
-  }
+static int launch_stats(rvk_volume* v, int frame, const void* dsrc) {
+  const int tasks = (v->nrb[0] + 7) / 8 * v->nrb[1] * v->nrb[2];
+  hipStream_t s = v->ctx->stream;
+  int* stats = v->frame_stats(frame);
+  if (sizeof(VT) == 2) hipLaunchKernelGGL(stats_init_kernel, dim3(1), dim3(kStatSlots), 0, s, stats);
+  hipLaunchKernelGGL((frame_stats_kernel<VT>), dim3((tasks + 3) / 4), dim3(256), 0, s, (const VT*)dsrc, v->dims[0],
+                     v->dims[1], v->dims[2], v->nrb[0], v->nrb[1], v->nrb[2], v->ranges[frame], stats);
+  RVK_HIP(hipGetLastError());
+  return RVK_OK;
 }
 
-template <typename VT>
-static int frame_range(rvk_volume* v, const void* dsrc, int& lo, int& hi, bool& odd_diff) {
-  const long long n = (long long)v->dims[0] * v->dims[1] * v->dims[2];
-  int* d = nullptr;
-  RVK_HIP(hipMallocAsync((void**)&d, 3 * sizeof(int), v->ctx->stream));
-  hipLaunchKernelGGL(range_init_kernel, dim3(1), dim3(64), 0, v->ctx->stream, d);
-  const int blocks = (int)std::min<long long>(4096, (n + 255) / 256);
-  hipLaunchKernelGGL((range_kernel<VT>), dim3(blocks), dim3(256), 0, v->ctx->stream, (const VT*)dsrc, n, v->dims[0],
-                     d);
-  int h[3] = {0, 0, 0};
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, v->ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(v->ctx->stream);
-  hipFreeAsync(d, v->ctx->stream);
-  if (e != hipSuccess) return hip_fail(e, "frame value range");
+static int frame_stats(rvk_volume* v, int frame, const void* dsrc, int& lo, int& hi, bool& odd_diff) {
+  if (!v->ranges[frame]) {
+    void* q = nullptr;
+    RVK_HIP(hipMalloc(&q, sizeof(float2) * v->n_range_bricks() + kStatBytes));
+    v->ranges[frame] = (float2*)q;
+  }
+  int rc = RVK_OK;
+  switch (v->dtype) {
+    case RVK_U8: return launch_stats<uint8_t>(v, frame, dsrc);
+    case RVK_I8: return launch_stats<int8_t>(v, frame, dsrc);
+    case RVK_U32: return launch_stats<uint32_t>(v, frame, dsrc);
+    case RVK_I32: return launch_stats<int32_t>(v, frame, dsrc);
+    case RVK_F32: return launch_stats<float>(v, frame, dsrc);
+    case RVK_U16: rc = launch_stats<uint16_t>(v, frame, dsrc); break;
+    default: rc = launch_stats<int16_t>(v, frame, dsrc); break;
+  }
+  if (rc) return rc;
+  int h[kStatSlots * kStatStride];
+  RVK_HIP(hipMemcpyAsync(h, v->frame_stats(frame), sizeof(h), hipMemcpyDeviceToHost, v->ctx->stream));
+  RVK_HIP(hipStreamSynchronize(v->ctx->stream));
   lo = h[0];
   hi = h[1];
   odd_diff = h[2] != 0;
+  for (int i = 1; i < kStatSlots; ++i) {
+    lo = std::min(lo, h[i * kStatStride]);
+    hi = std::max(hi, h[i * kStatStride + 1]);
+    odd_diff = odd_diff || h[i * kStatStride + 2] != 0;
+  }
   return RVK_OK;
 }
 
@@ -648,8 +720,8 @@ int rvk_volume_get_layout(const rvk_volume* v, int* layout) {
 }
 
 // Cells of one frame (in the volume's layout and the frame's encoding) from
-// x-fastest native voxels on the device, and (with_ranges) its range bricks.
-static int write_frame_cells(rvk_volume* v, int frame, const void* dsrc, bool with_ranges) {
+// x-fastest native voxels on the device.
+static int write_frame_cells(rvk_volume* v, int frame, const void* dsrc) {
   const int enc = v->enc[frame];
   // dispatched on the source voxel type: binary16 cells are written by the
   // difference relayout of their 16-bit source
@@ -657,23 +729,13 @@ static int write_frame_cells(rvk_volume* v, int frame, const void* dsrc, bool wi
   return dispatch_cells<false>(v->dtype, v->layout, half ? kEncDiff : enc, [&](auto tag) {
     using CV = decltype(tag);
     using VT = typename CV::value_type;
-    int r = RVK_OK;
     if constexpr (sizeof(VT) == 2 && CV::kDiff) {
-      if (enc == kEncHalfPair) r = launch_relayout<VT, CV::kLog2, true, 2>(v, dsrc, v->frames[frame]);
-      else if (enc == kEncHalf) r = launch_relayout<VT, CV::kLog2, true, 1>(v, dsrc, v->frames[frame]);
-      else r = launch_relayout<VT, CV::kLog2, true>(v, dsrc, v->frames[frame]);
+      if (enc == kEncHalfPair) return launch_relayout<VT, CV::kLog2, true, 2>(v, dsrc, v->frames[frame]);
+      if (enc == kEncHalf) return launch_relayout<VT, CV::kLog2, true, 1>(v, dsrc, v->frames[frame]);
+      return launch_relayout<VT, CV::kLog2, true>(v, dsrc, v->frames[frame]);
     } else {
-      r = launch_relayout<VT, CV::kLog2, CV::kDiff>(v, dsrc, v->frames[frame]);
+      return launch_relayout<VT, CV::kLog2, CV::kDiff>(v, dsrc, v->frames[frame]);
     }
-    if (r == RVK_OK && with_ranges) {
-      const int nb = v->nrb[0] * v->nrb[1] * v->nrb[2];
-      if (!v->ranges[frame]) RVK_HIP(hipMalloc((void**)&v->ranges[frame], sizeof(float2) * (size_t)nb));
-      hipLaunchKernelGGL((brick_range_kernel<VT>), dim3((nb + 255) / 256), dim3(256), 0, v->ctx->stream,
-                         (const VT*)dsrc, v->dims[0], v->dims[1], v->dims[2], v->nrb[0], v->nrb[1], v->nrb[2],
-                         v->ranges[frame]);
-      RVK_HIP(hipGetLastError());
-    }
-    return r;
   });
 }
 
@@ -773,7 +835,7 @@ int rvk_volume_relayout(rvk_volume* v, int layout) {
   }
   for (int f = 0; f < RVK_MAX_FRAMES && !rc; ++f) {
     if (!lin[f]) continue;
-    rc = write_frame_cells(v, f, lin[f], false);
+    rc = write_frame_cells(v, f, lin[f]);
     if (!rc && glin[f]) {
       if (v->layout == kCellLayoutBrick4) rc = launch_relayout<uint8_t, kCellLayoutBrick4>(v, glin[f], v->gradmag[f]);
       else if (v->layout == kCellLayoutPair8) rc = launch_relayout<uint8_t, kCellLayoutPair8>(v, glin[f], v->gradmag[f]);
@@ -809,13 +871,11 @@ int rvk_volume_set_frame(rvk_volume* v, int frame, const void* src, int src_on_d
   // frame's values span less than 32768 (then every difference fits), with
   // binary16 bases when they all lie in [-2048, 2048], and binary16
   // differences when these are exact too
-  int rc = RVK_OK;
   int enc = v->dtype == RVK_F32 ? kEncDiff : kEncPlain;
+  int lo = 0, hi = 0;
+  bool odd = false;
+  int rc = frame_stats(v, frame, dsrc, lo, hi, odd);
   if (v->dtype == RVK_U16 || v->dtype == RVK_I16) {
-    int lo = 0, hi = 0;
-    bool odd = false;
-    rc = v->dtype == RVK_U16 ? frame_range<uint16_t>(v, dsrc, lo, hi, odd)
-                             : frame_range<int16_t>(v, dsrc, lo, hi, odd);
     if (rc == RVK_OK && hi - lo <= 32767) {
       enc = kEncDiff;
       if (lo >= -2048 && hi <= 2048) enc = odd ? kEncHalf : kEncHalfPair;
@@ -823,7 +883,7 @@ int rvk_volume_set_frame(rvk_volume* v, int frame, const void* src, int src_on_d
   }
   if (rc == RVK_OK) {
     v->enc[frame] = (uint8_t)enc;
-    rc = write_frame_cells(v, frame, dsrc, true);
+    rc = write_frame_cells(v, frame, dsrc);
   }
   if (staging) {
     hipError_t e = hipStreamSynchronize(v->ctx->stream);

@@ -118,6 +118,50 @@ def test_drr_smallest_volumes_ragged_views(gpu_ctx, dims):
                 vh.close()
 
 
+@pytest.mark.parametrize("dims", [(62, 9, 7), (63, 7, 6), (64, 8, 15), (65, 17, 9), (130, 6, 10), (9, 66, 64)])
+def test_frame_statistics_at_the_edges_of_their_tiles(gpu_ctx, dims):
+    """The upload's value statistics (8-brick rows of 64 columns): a voxel
+    outside the binary16 range, or one odd x-neighbour difference above 2048,
+    decides the cell encoding wherever it lies, so an int16 volume with one
+    such voxel renders bit for bit as its float32 copy; and the range bricks
+    the batched march skips by leave its result that of the single-view one,
+    with a lone dense voxel in empty space at the same places."""
+    import torch
+    spacing = (1.0, 1.1, 0.9)
+    c = configs.volume_center(dims, spacing)
+    view = abi.compute_view(configs.drr_camera(c, 0.7, 24, sod=300.0, sid=600.0, fov=260.0, half_extent=130.0), 24, 40,
+                            spacing=spacing)
+    march = configs.march_params({"step_scale": 0.5, "term_T": 0.0, "jitter": 1, "skip_rule": 0})
+    drr = configs.drr_params({"intercept": 0.0, "slope": 1e-5, "offset": 1.0, "output": abi.DRR_F32_L,
+                              "ref_termination": 0})
+    rng = np.random.default_rng(dims[0])
+    at = sorted({(x, y, z) for x in (1, 6, 7, 8, 61, 62, 63, 64, dims[0] - 3, dims[0] - 2) if x < dims[0] - 1
+                 for y, z in ((1, 1), (dims[1] // 2, dims[2] // 2), (dims[1] - 2, dims[2] - 2))})
+    base = rng.integers(-40, 1400, dims[::-1]).astype(np.int16)
+    for x, y, z in at:
+        far = base.copy()
+        far[z, y, x] = 3000  # beyond +-2048
+        odd = base.copy()
+        odd[z, y, x], odd[z, y, x + 1] = -1000, 1501  # difference 2501
+        lone = np.zeros(dims[::-1], np.int16)
+        lone[z, y, x] = 1500
+        for vol in (far, odd, lone):
+            got = []
+            for v in (vol, vol.astype(np.float32)):
+                vh = H.gpu_volume(gpu_ctx, v, spacing)
+                out = torch.full((view.height, view.width), float("nan"), dtype=torch.float32, device="cuda")
+                abi.render_drr(gpu_ctx, vh, view, march, drr, out)
+                plan = abi.DrrPlan(gpu_ctx, vh, [view], march, drr)
+                batched = torch.full((plan.total,), float("nan"), dtype=torch.float32, device="cuda")
+                plan.render(batched)
+                torch.cuda.synchronize()
+                got += [out.cpu().numpy().ravel(), batched.cpu().numpy()]
+                plan.close()
+                vh.close()
+            assert np.isfinite(got[0]).all()
+            assert all(np.array_equal(got[0], g) for g in got[1:]), (x, y, z)
+
+
 @pytest.mark.parametrize("dtype", ["u16", "i16"])
 def test_drr_wide_range_16bit_frames(gpu_ctx, dtype):
     """16-bit frames whose values span 32768 or more keep plain (a, b) cells
