@@ -16,68 +16,10 @@
 #include <cstring>
 #include <vector>
 
-#include "rvk_internal.h"
-#include "rvk_march.h"
+#include "rvk_lanes.h"
 #include "rvk_pose_math.h"
 
 namespace rvk {
-
-struct BatchView {
-  ViewGeom v;
-  float dm[96];      // d(view_to_voxels)/d pose_i, i = 0..5 (baked, row major)
-  float inv[16];     // inverse of view_to_voxels: voxel position -> (vx, vy, z, 1) * w
-  long long pix_off; // first pixel of this view in the packed image buffer
-  int tiles16_x;
-  int pad;
-};
-
-struct BatchArgs {
-  VolGeom g;
-  DrrMarchArgs m;
-  float step_len;
-  const void* vol;
-  const BatchView* views;
-  const int* item_begin;  // n_views + 1 prefix sums of 8x8 tiles
-  int n_views;
-  int n_items;
-  float* out;
-  float* jac;             // 6 x total pixels (SoA) d L_p / d pose_i, or NULL
-  long long total;        // pixels in the packed images
-  unsigned* queues;       // kNumXcd work-queue heads (persistent schedule)
-  int shape;              // wave tile of the forward kernels (RVK_TILE_*)
-  const int2* work;       // forward work order: (view, tile of the view) per work item
-};
-
-// Accumulates S = sum grad mu and T = sum (j+t) grad mu over the accumulated
-// samples of one ray; A = ds*slope*S and B = ds*slope*T (see the pose adjoint
-// below) are formed once per ray by pose_sums().
-struct PoseVisit {
-  static constexpr bool kFlatRuns = true;  // a zero gradient adds nothing
-  float j;
-  V3<float>& S;
-  V3<float>& T;
-  __device__ __forceinline__ void operator()(const V3<float>&, float t, float, const V3<float>& gr) const {
-    const float w = j + t;
-    S.x += gr.x; S.y += gr.y; S.z += gr.z;
-    T.x = fmaf(w, gr.x, T.x); T.y = fmaf(w, gr.y, T.y); T.z = fmaf(w, gr.z, T.z);
-  }
-};
-// Scales the sums by ncs = ds*slope; called only for rays that accumulated
-// a sample (a ray that misses the volume can have a non-finite ds).
-__device__ __forceinline__ void pose_sums(float ncs, V3<float>& A, V3<float>& B) {
-  A.x *= ncs; A.y *= ncs; A.z *= ncs;
-  B.x *= ncs; B.y *= ncs; B.z *= ncs;
-}
-
-__device__ __forceinline__ int find_view(const int* __restrict__ ib, int n, int item) {
-  int lo = 0, hi = n;  // ib[lo] <= item < ib[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (ib[mid] <= item) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
 
 __device__ __forceinline__ void item_pixel(int tiles16_x, int local, int lane, int& x, int& y) {
   const int macro = local >> 2, q = local & 3;
@@ -143,7 +85,7 @@ __device__ __forceinline__ void forward_item(const BatchArgs& a, int item, int l
 // One wave per tile; workgroups XCD-remapped so neighbouring tiles share an L2.
 template <typename CV, bool SKIP, bool PRECISE, bool JAC, bool TERM>
 __global__ __launch_bounds__(256) void batch_grid_kernel(BatchArgs a) {
-  const int blk = xcd_remap(blockIdx.x, gridDim.x);
+  const int blk = a.deal ? xcd_deal(blockIdx.x, kDealLog2) : xcd_remap(blockIdx.x, gridDim.x);
   const int item = blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (item >= a.n_items) return;
   forward_item<CV, SKIP, PRECISE, JAC, TERM>(a, item, threadIdx.x & 63);
@@ -195,15 +137,6 @@ struct NccArgs {
   float* loss;     // n_views
   float* grad_img; // optional packed dloss/dI
 };
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
-}
-__device__ __forceinline__ float wave_sumf(float v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
-}
 
 __global__ __launch_bounds__(256) void ncc_partial_kernel(NccArgs a) {
   const int item = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -257,11 +190,6 @@ __global__ __launch_bounds__(256) void ncc_view_kernel(NccArgs a) {
   }
 }
 
-// d loss / d I_p = -( (T_p - mean_T) / sqrt(Saa Sbb) - ncc (I_p - mean_I) / Saa )
-__device__ __forceinline__ float dloss_dimage(const double* st, float I, float T) {
-  return (float)(-((double)T - st[1]) * st[2] + st[3] * ((double)I - st[0]));
-}
-
 __global__ __launch_bounds__(256) void ncc_grad_image_kernel(NccArgs a) {
   const int item = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (item >= a.n_items) return;
@@ -275,38 +203,17 @@ __global__ __launch_bounds__(256) void ncc_grad_image_kernel(NccArgs a) {
   a.grad_img[i] = dloss_dimage(a.stats + 8 * v, a.img[i], a.tgt[i]);
 }
 
-// ---------------------------------------------------------------------------
-// Pose adjoint.  For one pixel, L = sum_m ds*mu(p_m) over accumulated samples
-// p_m = start + (j + t_m) inc, so
-//   dL/dpose_i = A . dstart_i + B . dinc_i,
-//   A = sum_m ds*slope*grad mu(p_m),   B = sum_m (j + t_m) ds*slope*grad mu(p_m),
-// with (dstart_i, dinc_i) the forward-mode tangent of the ray set-up along
-// d(view_to_voxels)/d pose_i.  The ray is re-marched (PRECISE positions) with
-// the forward's control flow; nothing is stored per sample.
-struct AdjArgs {
-  BatchArgs b;
-  const float* img;   // rendered images (packed)
-  const float* dldi;  // d loss / d image, or NULL: formed from the NCC state
-  const double* stats;
-  const float* tgt;
-  float* part;  // n_items x 6
-};
-
-__device__ __forceinline__ float dloss_at(const float* dldi, const double* stats, const float* img, const float* tgt,
-                                          int v, long long pi) {
-  return dldi ? dldi[pi] : dloss_dimage(stats + 8 * v, img[pi], tgt[pi]);
-}
-
-template <typename CV, bool SKIP>
+template <typename CV, bool SKIP, bool TERM>
 __global__ __launch_bounds__(256) void adjoint_pose_kernel(AdjArgs a) {
-  const int blk = xcd_remap(blockIdx.x, gridDim.x);
+  const int blk = a.b.deal ? xcd_deal(blockIdx.x, kDealLog2) : xcd_remap(blockIdx.x, gridDim.x);
   const int item = blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (item >= a.b.n_items) return;
   const int lane = threadIdx.x & 63;
-  const int v = __builtin_amdgcn_readfirstlane(find_view(a.b.item_begin, a.b.n_views, item));
+  const int2 vt = a.b.work[item];
+  const int v = __builtin_amdgcn_readfirstlane(vt.x), local = __builtin_amdgcn_readfirstlane(vt.y);
   const BatchView& bv = a.b.views[v];
   int x, y;
-  item_pixel(bv.tiles16_x, item - a.b.item_begin[v], lane, x, y);
+  item_pixel(bv.tiles16_x, local, lane, x, y);
   float c[6] = {0, 0, 0, 0, 0, 0};
   if (x < bv.v.W && y < bv.v.H) {
     const VolGeom& g = a.b.g;
@@ -316,7 +223,7 @@ __global__ __launch_bounds__(256) void adjoint_pose_kernel(AdjArgs a) {
     V3<float> A{0, 0, 0}, B{0, 0, 0};
     const float jt = ray_offset(a.b.m.jitter, x, y);
     PoseVisit visit{jt, A, B};
-    const float I = drr_march<CV, SKIP, true, true, true>(cells_of<CV>(a.b.vol), g, a.b.m, r, x, y, visit);
+    const float I = drr_march<CV, SKIP, true, true, true, true, TERM>(cells_of<CV>(a.b.vol), g, a.b.m, r, x, y, visit);
     const long long pi = bv.pix_off + (long long)y * bv.v.W + x;
     const float dLdI = dloss_at(a.dldi, a.stats, a.img, a.tgt, v, pi);
     // dI/dL = -I for exp(-L) output, 1 for L output
@@ -335,7 +242,7 @@ __global__ __launch_bounds__(256) void adjoint_pose_kernel(AdjArgs a) {
   for (int i = 0; i < 6; ++i) c[i] = wave_sumf(c[i]);
   if (lane == 0)
 #pragma unroll
-    for (int i = 0; i < 6; ++i) a.part[(long long)item * 6 + i] = c[i];
+    for (int i = 0; i < 6; ++i) a.part[((long long)a.b.item_begin[v] + local) * 6 + i] = c[i];
 }
 
 __global__ __launch_bounds__(256) void pose_reduce_kernel(const int* item_begin, const float* part, float* grad) {
@@ -781,6 +688,7 @@ struct rvk_drr_plan {
   // an XCD's L2 serves one region's cells to every view)
   int2* d_work[2] = {nullptr, nullptr};
   int order = 0, jac_order = 0;
+  bool auto_order = true;  // no order set or tuned yet
   // the fused registration forward (pose Jacobians) has its own schedule:
   // its per-wave work differs enough that the best choice can differ
   int jac_schedule = RVK_SCHED_GRID;
@@ -906,6 +814,20 @@ static int upload_work_orders(rvk_drr_plan* p, const rvk_view* views) {
   return RVK_OK;
 }
 
+// The order the marches take the tiles in: the plan's, or until one is set or
+// tuned the region order with its tiles dealt to the XCDs in runs of 8.  The
+// regions cluster what the views share, and the deal evens out what the runs
+// leave each XCD to do (us, forward / pose adjoint): 64 poses of a 512x512x400
+// CT 25100 / 35250 view by view in bands, 21310 / 31790 so, 4 poses 2996 / 3443
+// and 1706 / 2436; 16 x 512^2 half a circle around a 256^3 f32 volume
+// 1683 / 1809 and 1590 / 1741.  Dealing the view-major order is slower there
+// (2500 / 2800: the XCDs then share no view's cells).
+void use_order(const rvk_drr_plan* p, BatchArgs& a, int order) {
+  const bool regions = p->auto_order || order == RVK_ORDER_REGIONS;
+  a.work = p->d_work[regions ? 1 : 0];
+  a.deal = regions;
+}
+
 BatchArgs batch_args(const rvk_drr_plan* p, float* out) {
   BatchArgs a;
   a.g = vol_geom(p->vol);
@@ -916,6 +838,9 @@ BatchArgs batch_args(const rvk_drr_plan* p, float* out) {
   a.m.ranges = p->vol->ranges[p->frame];
   a.m.rbx = p->vol->nrb[0];
   a.m.rby = p->vol->nrb[1];
+  a.m.groups = p->vol->range_groups(p->frame);
+  a.m.rgx = p->vol->nrg(0);
+  a.m.rgy = p->vol->nrg(1);
   a.m.ref_term = p->drr.ref_termination;
   a.m.jitter = p->march.jitter;
   a.step_len = min_spacing(p->vol) * p->march.step_scale;
@@ -929,15 +854,25 @@ BatchArgs batch_args(const rvk_drr_plan* p, float* out) {
   a.total = p->pix_off[p->n_views];
   a.queues = p->d_queues;
   a.shape = p->shape;
-  a.work = p->d_work[p->order];
+  use_order(p, a, p->order);
   return a;
+}
+
+// log2 of the lanes per ray of the plan's forward (grad: with Jacobians).  A
+// march that may terminate takes one.
+int plan_lanes(const rvk_drr_plan* p, bool grad) {
+  if (p->drr.ref_termination) return 0;
+  return batch_lanes(p->vol, p->pix_off[p->n_views], min_spacing(p->vol) * p->march.step_scale, grad);
 }
 
 int launch_forward(rvk_drr_plan* p, float* out, hipStream_t s, bool jac = false) {
   BatchArgs a = batch_args(p, out);
   a.shape = jac ? p->jac_shape : p->shape;
-  a.work = p->d_work[jac ? p->jac_order : p->order];
+  use_order(p, a, jac ? p->jac_order : p->order);
   const bool skip = p->march.skip_rule != 0, pr = p->march.precise != 0;
+  // several lanes per ray are part of the default schedule and tile
+  if ((pr || jac) && a.shape == RVK_TILE_8X8 && (jac ? p->jac_schedule : p->schedule) == RVK_SCHED_GRID)
+    if (const int ls = plan_lanes(p, jac)) return launch_batch_lanes(a, p->vol, p->frame, skip, jac, ls, s);
   return dispatch_frame(p->vol, p->frame, [&](auto tag) {
     using CV = decltype(tag);
     const int sched = jac ? p->jac_schedule : p->schedule;
@@ -957,7 +892,7 @@ int launch_forward(rvk_drr_plan* p, float* out, hipStream_t s, bool jac = false)
       else { if (pr) RVK_LP(false, true, false); else RVK_LP(false, false, false); }
 #undef RVK_LP
     } else {
-      const int blocks = (p->n_items + 3) / 4;
+      const unsigned blocks = batch_grid(a, 0);
 #define RVK_LG(S, P, J)                                                                                     \
   do {                                                                                                      \
     if (p->drr.ref_termination)                                                                             \
@@ -1200,6 +1135,7 @@ int rvk_drr_plan_autotune(rvk_drr_plan* p, float* out, int reps, float* best_ms)
   reps = std::max(1, std::min(reps, 100));
   RVK_HIP(hipSetDevice(p->ctx->device));
   drop_graph(p);
+  p->auto_order = false;
   // schedule x waves per SIMD x wave tile x work order
   const int cand[][2] = {{RVK_SCHED_GRID, 4}, {RVK_SCHED_PERSISTENT, 2}, {RVK_SCHED_PERSISTENT, 4},
                          {RVK_SCHED_PERSISTENT, 8}};
@@ -1298,7 +1234,8 @@ int rvk_drr_plan_set_work_order(rvk_drr_plan* p, int order) {
   if (!p) return fail(RVK_ERR_INVALID_ARGUMENT, "plan is NULL");
   if (order != RVK_ORDER_VIEWS && order != RVK_ORDER_REGIONS)
     return fail(RVK_ERR_INVALID_ARGUMENT, "unknown work order %d", order);
-  if (order != p->order || order != p->jac_order) drop_graph(p);
+  if (p->auto_order || order != p->order || order != p->jac_order) drop_graph(p);
+  p->auto_order = false;
   p->order = p->jac_order = order;
   return RVK_OK;
 }
@@ -1405,8 +1342,17 @@ int rvk_drr_plan_backward(rvk_drr_plan* p, const float* images, const float* dld
     aa.part = p->d_pose_part;
     int rc = dispatch_frame(p->vol, p->frame, [&](auto tag) {
       using CV = decltype(tag);
-      if (p->march.skip_rule) hipLaunchKernelGGL((adjoint_pose_kernel<CV, true>), dim3(blocks), dim3(256), 0, s, aa);
-      else hipLaunchKernelGGL((adjoint_pose_kernel<CV, false>), dim3(blocks), dim3(256), 0, s, aa);
+#define RVK_LA(S)                                                                                            \
+  do {                                                                                                       \
+    if (p->drr.ref_termination)                                                                              \
+      hipLaunchKernelGGL((adjoint_pose_kernel<CV, S, true>), dim3(blocks), dim3(256), 0, s, aa);             \
+    else                                                                                                     \
+      hipLaunchKernelGGL((adjoint_pose_kernel<CV, S, false>), dim3(blocks), dim3(256), 0, s, aa);            \
+  } while (0)
+      const unsigned blocks = batch_grid(aa.b, 0);
+      if (p->march.skip_rule) RVK_LA(true);
+      else RVK_LA(false);
+#undef RVK_LA
       return (int)RVK_OK;
     });
     if (rc) return rc;

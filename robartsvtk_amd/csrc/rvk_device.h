@@ -810,6 +810,20 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblk) {
   return (xcd < rem) ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
 }
 
+// Tiles dealt to the XCDs in runs of 2^run_log2 consecutive ones, run i to XCD
+// i mod 8, instead of one band per XCD: a march that passes over empty space
+// makes the bands through it cheap and the body's expensive, and the XCDs of
+// the cheap ones would idle.  The grid is a multiple of 8 runs (deal_grid).
+__device__ __forceinline__ int xcd_deal(int bid, int run_log2) {
+  const int xcd = bid % kNumXcd, local = bid / kNumXcd;
+  return (((local >> run_log2) * kNumXcd + xcd) << run_log2) + (local & ((1 << run_log2) - 1));
+}
+constexpr int kDealLog2 = 3;  // runs of 8 workgroups
+inline unsigned deal_grid(long long nblk, int run_log2) {
+  const long long m = (long long)kNumXcd << run_log2;
+  return (unsigned)((nblk + m - 1) / m * m);
+}
+
 // 16x16-pixel workgroup tiles are ordered in super-tiles of 2^kSuperLog2 x
 // 2^kSuperLog2 tiles (row-major over super-tiles, row-major inside), so the
 // tiles an XCD runs at one time cover a compact image region (and volume
@@ -819,14 +833,17 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblk) {
 #define RVK_SUPER_LOG2 2
 #endif
 constexpr int kSuperLog2 = RVK_SUPER_LOG2;
+__device__ __forceinline__ void tile_origin(int tile, int stiles_x, int& px, int& py) {
+  const int st = tile >> (2 * kSuperLog2), in = tile & ((1 << (2 * kSuperLog2)) - 1);
+  px = ((st % stiles_x) * (1 << kSuperLog2) + (in & ((1 << kSuperLog2) - 1))) * 16;
+  py = ((st / stiles_x) * (1 << kSuperLog2) + (in >> kSuperLog2)) * 16;
+}
 __device__ __forceinline__ void tile_pixel(int tile, int stiles_x, int& px, int& py) {
   const int t = threadIdx.x;
   const int w = t >> 6, l = t & 63;
-  const int st = tile >> (2 * kSuperLog2), in = tile & ((1 << (2 * kSuperLog2)) - 1);
-  const int tx = (st % stiles_x) * (1 << kSuperLog2) + (in & ((1 << kSuperLog2) - 1));
-  const int ty = (st / stiles_x) * (1 << kSuperLog2) + (in >> kSuperLog2);
-  px = tx * 16 + (w & 1) * 8 + (l & 7);
-  py = ty * 16 + (w >> 1) * 8 + (l >> 3);
+  tile_origin(tile, stiles_x, px, py);
+  px += (w & 1) * 8 + (l & 7);
+  py += (w >> 1) * 8 + (l >> 3);
 }
 
 }  // namespace rvk

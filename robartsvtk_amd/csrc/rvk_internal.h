@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -37,8 +38,12 @@ struct rvk_volume {
   // allocation ends with the totals an upload collects (frame_stats).
   float2* ranges[RVK_MAX_FRAMES] = {};
   int nrb[3] = {0, 0, 0};
+  // The same of every 4^3 range bricks follows in the allocation.
   size_t n_range_bricks() const { return (size_t)nrb[0] * nrb[1] * nrb[2]; }
-  int* frame_stats(int f) const { return reinterpret_cast<int*>(ranges[f] + n_range_bricks()); }
+  int nrg(int a) const { return (nrb[a] + 3) / 4; }
+  size_t n_range_groups() const { return (size_t)nrg(0) * nrg(1) * nrg(2); }
+  float2* range_groups(int f) const { return ranges[f] ? ranges[f] + n_range_bricks() : nullptr; }
+  int* frame_stats(int f) const { return reinterpret_cast<int*>(ranges[f] + n_range_bricks() + n_range_groups()); }
   // bumped whenever the frames' cells move (rvk_volume_relayout): graphs
   // captured before hold stale cell pointers and are not replayed
   unsigned generation = 0;
@@ -168,6 +173,13 @@ inline int check_march(const rvk_march_params* m) {
   if (!(m->step_scale > 0.0f) || !(m->step_scale < __builtin_huge_valf()))
     return fail(RVK_ERR_INVALID_ARGUMENT, "step_scale must be positive and finite");
   return RVK_OK;
+}
+
+// Samples along the longest axis of the volume.
+inline float longest_ray(const rvk_volume* v, float step_len) {
+  double m = 0.0;
+  for (int a = 0; a < 3; ++a) m = std::max(m, v->dims[a] * v->spacing[a]);
+  return (float)(m / step_len);
 }
 
 // Workgroups for a caster launch over a view: whole super-tiles of

@@ -1,0 +1,54 @@
+// rvk_lanes.h -- how a DRR launch spreads its rays, and the kernels with
+// several lanes on one ray (rvk_lanes.hip).
+#pragma once
+#include "rvk_batch.h"
+
+namespace rvk {
+
+// The schedule of a precise march without termination.
+struct DrrSchedule {
+  int lanes;  // log2 of the lanes per ray
+  bool deal;  // tiles dealt to the XCDs in runs (xcd_deal), or one band each
+  bool runs;  // pass over runs of empty and constant bricks
+};
+
+// One view of `rays` rays.  The device holds 8192 waves, and 64 rays are one
+// wave: below about 600 thousand rays it waits on chains of dependent
+// samples, which more lanes per ray shorten; the chunks' bookkeeping costs
+// throughput above.  Measured (us, skip rule, int16 CT, 1 / 2 / 4 / 8 / 16
+// lanes): 256^3 of 512-sample rays at 64^2 261 / 157 / 80 / 43 / 24, 128^2
+// 265 / 159 / 83 / 48 / 38, 360^2 208 / 137 / 91 / -, 512^2 262 / 191 / 180 / -,
+// 724^2 236 / 254 / 274, 1024^2 360 / 426 / 480; 400^3 724^2 368 / 316 / 358;
+// 128^3 of 128-sample rays at 128^2 64 / 40 / 23 / 15 / 12, 360^2 60 / 44 / 41 / 43,
+// 512^2 53 / 63 / 59.  Short rays have no runs worth finding (128^3 at 200^2
+// 24 us without, 36 with) and share their cells within an XCD's band, and so
+// does the smallest launch (256^3 at 64^2: 24 us without runs, 29 with).
+inline DrrSchedule drr_schedule(const rvk_volume* vol, long long rays, float step_len) {
+  if (rays <= 24576) return {4, false, false};
+  if (longest_ray(vol, step_len) >= 192.0f) return {rays <= 300000 ? 2 : rays <= 600000 ? 1 : 0, true, true};
+  return rays <= 200000 ? DrrSchedule{2, false, false} : DrrSchedule{0, false, true};
+}
+
+// log2 of the lanes per ray for a plan's forward of `rays` rays in all (in its
+// grid schedule), always with runs.  grad: the march also sums gradients, and every lane forms the ray's set-up and shares its tangents,
+// so more lanes pay less.  Measured (us, register on f32 / int16 volumes,
+// 1 / 2 / 4 / 8 / 16 lanes): 200^3 1 x 128^2 133 / 78 / 51 / 40 / 39, 2 x 128^2
+// 139 / 82 / 57 / 53 / 63, 2 x 200^2 151 / 92 / 74 / 77 / 84, 8 x 200^2
+// 266 / 198 / 195 / 218, 4 x 400^2 211 / 213 / 260, 8 x 400^2 325 / 357; 256^3 (512
+// samples) 8 x 200^2 610 / 406 / 362 / 389, 8 x 400^2 793 / 661 / 735, 16 x 512^2
+// 1855 / 1931; its plain render 1590 / 1359 / 1629.
+inline int batch_lanes(const rvk_volume* vol, long long rays, float step_len, bool grad) {
+  if (rays <= 24576) return 4;
+  if (rays <= 49152) return 3;
+  if (rays <= 400000) return 2;
+  const bool is_long = longest_ray(vol, step_len) >= 256.0f;
+  return rays <= (!is_long ? 700000 : grad ? 1500000 : 4500000) ? 1 : 0;
+}
+
+// One view; nblk is the launch's count of 16x16-pixel tiles (launch_grid).
+int launch_drr_lanes(const DrrArgs& a, const rvk_volume* vol, int frame, bool skip, int ls, int nblk, hipStream_t s);
+// A plan's forward (jac: with the pose Jacobians).
+int launch_batch_lanes(const BatchArgs& a, const rvk_volume* vol, int frame, bool skip, bool jac, int ls,
+                       hipStream_t s);
+
+}  // namespace rvk

@@ -108,87 +108,116 @@ struct DrrMarchArgs {
   int output, ref_term, jitter;
   const float2* ranges;  // per range brick (min, max) of the frame, or NULL
   int rbx, rby;          // range-brick grid extent in x and y
+  const float2* groups;  // the same per 4^3 range bricks
+  int rgx, rgy;
+};
+
+// One view of the single-view caster.
+struct DrrArgs {
+  VolGeom g;
+  ViewGeom v;
+  float step_len;
+  DrrMarchArgs m;
+  uint32_t tint;
+  const void* vol;
+  void* out;
+  int tiles_x;
+  int deal;  // tiles dealt to the XCDs in runs (xcd_deal), or one band each
 };
 
 // Run skipping of the precise march.  Each range brick (kRangeEdge^3 cells)
-// has the (min, max) of every value its cells can interpolate.  After a
-// sample at cell coordinate q:
-//  - if no value of q's brick can contribute (alpha = fma(cs, v, ci) >= 0 at
-//    the bound that minimises it: alpha is monotone in v), the samples the
-//    march takes next inside the brick do not contribute either;
-//  - if the brick is constant (min == max: every corner equal, so every
-//    sample in it interpolates that value exactly) and q contributed, the
-//    next samples contribute the same alpha.
+// has the (min, max) of every value its cells can interpolate, and each group
+// of 4^3 bricks (32^3 cells) that of its bricks.  After a sample at cell
+// coordinate q, with R the group that holds q, or else its brick:
+//  - if no value of R can contribute (alpha = fma(cs, v, ci) >= 0 at the
+//    bound that minimises it: alpha is monotone in v), the samples the march
+//    takes next inside R do not contribute either;
+//  - if R is constant (min == max: every corner equal, so every sample in it
+//    interpolates that value exactly) and q contributed, the next samples
+//    contribute the same alpha.
 // Either way the march's state after such a run is known in closed form, so
-// the run's gathers are skipped (a contributing run still adds its alphas
-// one by one, in order: the sum is the same to the bit).
+// the run's gathers are skipped (a contributing run of m adds m alpha with
+// one f64 rounding; with termination it adds one by one, testing each).
+//
+// The run ends kRunMargin voxels before R's far face, so that no rounding of
+// the exit time or of a sample's position (below 0.0015 voxels for coordinates
+// up to 4097) can count a sample outside R; positions are monotone in t.
+constexpr float kRunMargin = 0.004f;
 struct RangeWalk {
-  float hx, hy, hz;  // the brick face a ray leaves through: kRangeEdge (ahead) or 0
-  float rx, ry, rz;  // 1 / inc, +inf where inc = 0
+  V3<float> e, c;     // exit time of the brick with index b on an axis: b e + c
+  V3<uint32_t> far;   // 3 on axes the ray goes up: a group's last brick is b | 3, else b & ~3
 };
-__device__ __forceinline__ RangeWalk range_walk(const V3<float>& inc) {
-  const float e = (float)kRangeEdge, inf = __builtin_huge_valf();
-  return RangeWalk{inc.x >= 0.0f ? e : 0.0f, inc.y >= 0.0f ? e : 0.0f, inc.z >= 0.0f ? e : 0.0f,
-                   inc.x != 0.0f ? 1.0f / inc.x : inf, inc.y != 0.0f ? 1.0f / inc.y : inf,
-                   inc.z != 0.0f ? 1.0f / inc.z : inf};
+__device__ __forceinline__ RangeWalk range_walk(const V3<float>& p0c, const V3<float>& inc) {
+  RangeWalk w;
+  auto axis = [](float p, float i, float& e, float& c, uint32_t& far) {
+    const float r = 1.0f / i;
+    e = i != 0.0f ? (float)kRangeEdge * r : 0.0f;
+    c = i != 0.0f ? ((i > 0.0f ? (float)kRangeEdge - kRunMargin : kRunMargin) - p) * r : __builtin_huge_valf();
+    far = i > 0.0f ? 3u : 0u;
+  };
+  axis(p0c.x, inc.x, w.e.x, w.c.x, w.far.x);
+  axis(p0c.y, inc.y, w.e.y, w.c.y, w.far.y);
+  axis(p0c.z, inc.z, w.e.z, w.c.z, w.far.z);
+  return w;
 }
 
-// How many of the samples t1, t1 + stride, ... before lim lie in range brick
-// (bx, by, bz), which holds the sample before t1.  The estimate from the
-// brick's exit time is confirmed on its last sample, at the exact position
-// the march computes: positions are monotone in t per axis, so when the
-// sample before t1 and the last one lie in the (box-shaped) brick, all
-// between do.  t1 and lim are integers, so the cap at lim is exact.
-__device__ __forceinline__ int brick_run(int bx, int by, int bz, const V3<float>& p0c, const V3<float>& inc,
-                                         const RangeWalk& w, float t1, float lim, float stride) {
-  const float e = (float)kRangeEdge;
-  const float tx = (fmaf((float)bx, e, w.hx) - p0c.x) * w.rx;
-  const float ty = (fmaf((float)by, e, w.hy) - p0c.y) * w.ry;
-  const float tz = (fmaf((float)bz, e, w.hz) - p0c.z) * w.rz;
+// The ranges around q and the brick index; group = whether `use` holds for
+// the group's range, and the return whether for either.
+struct RangeAt {
+  uint32_t bx, by, bz;
+  bool group;
+};
+template <typename U>
+__device__ __forceinline__ bool range_at(const DrrMarchArgs& a, const V3<float>& q, RangeAt& at, U&& use) {
+  at.bx = (uint32_t)(int)q.x >> kRangeLog2;
+  at.by = (uint32_t)(int)q.y >> kRangeLog2;
+  at.bz = (uint32_t)(int)q.z >> kRangeLog2;
+  const float2 g = a.groups[((at.bz >> 2) * (uint32_t)a.rgy + (at.by >> 2)) * (uint32_t)a.rgx + (at.bx >> 2)];
+  const float2 r = a.ranges[(at.bz * (uint32_t)a.rby + at.by) * (uint32_t)a.rbx + at.bx];
+  at.group = use(g);
+  return at.group || use(r);
+}
+
+// How many of the samples t1, t1 + stride, ... before lim (stride a power of
+// two; t1 and lim integers) lie in the region, which holds the sample before.
+__device__ __forceinline__ float run_length(const RangeAt& at, const RangeWalk& w, float t1, float lim,
+                                            float inv_stride) {
+  const uint32_t keep = at.group ? ~3u : ~0u, on = at.group ? 3u : 0u;
+  const float tx = fmaf((float)((at.bx & keep) | (w.far.x & on)), w.e.x, w.c.x);
+  const float ty = fmaf((float)((at.by & keep) | (w.far.y & on)), w.e.y, w.c.y);
+  const float tz = fmaf((float)((at.bz & keep) | (w.far.z & on)), w.e.z, w.c.z);
   const float te = fminf(fminf(tx, ty), fminf(tz, lim));
-  const float inv = stride == 1.0f ? 1.0f : 0.5f;
-  int m = (int)ceilf((te - t1) * inv);
-  for (int k = 0; k < 2 && m > 0; ++k, --m) {
-    const float tl = fmaf(stride, (float)(m - 1), t1);
-    const int cx = (int)fmaf(tl, inc.x, p0c.x), cy = (int)fmaf(tl, inc.y, p0c.y), cz = (int)fmaf(tl, inc.z, p0c.z);
-    if ((cx >> kRangeLog2) == bx && (cy >> kRangeLog2) == by && (cz >> kRangeLog2) == bz) return m;
-  }
-  return 0;
-}
-
-__device__ __forceinline__ float2 range_brick(const DrrMarchArgs& a, const V3<float>& q, int& bx, int& by, int& bz) {
-  bx = (int)q.x >> kRangeLog2;
-  by = (int)q.y >> kRangeLog2;
-  bz = (int)q.z >> kRangeLog2;
-  return a.ranges[(bz * a.rby + by) * a.rbx + bx];
+  return fmaxf(ceilf((te - t1) * inv_stride), 0.0f);
 }
 
 // Non-contributing samples to pass over after the one at q (the next at t1).
-__device__ __forceinline__ int empty_run(const DrrMarchArgs& a, const V3<float>& q, const V3<float>& p0c,
-                                         const V3<float>& inc, const RangeWalk& w, float cs, float ci, float t1,
-                                         float lim, float stride) {
-  int bx, by, bz;
-  const float2 r = range_brick(a, q, bx, by, bz);
-  if (!(fmaf(cs, cs <= 0.0f ? r.y : r.x, ci) >= 0.0f)) return 0;
-  return brick_run(bx, by, bz, p0c, inc, w, t1, lim, stride);
+__device__ __forceinline__ float empty_run(const DrrMarchArgs& a, const V3<float>& q, const RangeWalk& w, float cs,
+                                           float ci, float t1, float lim, float inv_stride) {
+  RangeAt at;
+  if (!range_at(a, q, at, [&](const float2& r) { return fmaf(cs, cs <= 0.0f ? r.y : r.x, ci) >= 0.0f; }))
+    return 0.0f;
+  return run_length(at, w, t1, lim, inv_stride);
 }
 
 // Contributing run after the sample at q (alpha; next sample at t): adds the
 // run's alphas to acc and advances t.  Returns true when acc reached stop_at
 // inside the run (the march ends there, as it would have).
-template <typename Acc>
-__device__ __forceinline__ bool flat_run(const DrrMarchArgs& a, const V3<float>& q, const V3<float>& p0c,
-                                         const V3<float>& inc, const RangeWalk& w, float cs, float ci, float alpha,
-                                         float& t, float lim, Acc& acc, Acc stop_at) {
-  int bx, by, bz;
-  const float2 r = range_brick(a, q, bx, by, bz);
-  if (!(r.x == r.y && fmaf(cs, r.x, ci) == alpha)) return false;
-  const int m = brick_run(bx, by, bz, p0c, inc, w, t, lim, 1.0f);
-  for (int i = 0; i < m; ++i) {
-    acc += (Acc)alpha;
-    if (acc <= stop_at) return true;
+template <bool TERM, typename Acc>
+__device__ __forceinline__ bool flat_run(const DrrMarchArgs& a, const V3<float>& q, const RangeWalk& w, float cs,
+                                         float ci, float alpha, float& t, float lim, float stride, float inv_stride,
+                                         Acc& acc, Acc stop_at) {
+  RangeAt at;
+  if (!range_at(a, q, at, [&](const float2& r) { return r.x == r.y && fmaf(cs, r.x, ci) == alpha; })) return false;
+  const float m = run_length(at, w, t, lim, inv_stride);
+  if (TERM) {
+    for (int i = 0; i < (int)m; ++i) {
+      acc += (Acc)alpha;
+      if (acc <= stop_at) return true;
+    }
+  } else {
+    acc = fma((Acc)m, (Acc)alpha, acc);
   }
-  t += (float)m;
+  t = fmaf(m, stride, t);
   return false;
 }
 
@@ -198,6 +227,16 @@ struct NoVisit {
   static constexpr bool kFlatRuns = true;
   __device__ __forceinline__ void operator()(const V3<float>&, float, float, const V3<float>&) const {}
 };
+
+// The output of a march that ended with accumulator L, by selects: written as
+// a chain of uniform branches, hipcc's code for the L output skipped the
+// negation in some of the kernels this is inlined into.
+__device__ __forceinline__ float drr_value(const DrrMarchArgs& a, float L) {
+  const float e = expf(L), o = 256.0f - e;
+  const float ref = o < 0.0f ? 0.0f : o;
+  const float v = a.output == RVK_DRR_F32_EXP_NEG_L ? e : -L;
+  return a.output == RVK_DRR_RGBA8_REF ? ref : v;
+}
 
 // Line integral along one ray.  The accumulator starts at ln(256*offset) in
 // the reference RGBA8 mode and at 0 in the float modes.  `visit(c, t, alpha,
@@ -244,7 +283,7 @@ __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMa
   // updates one float in place
   float z = 0.0f;
   const bool runs = RUNS && PRECISE && a.ranges != nullptr;
-  const RangeWalk w = range_walk(inc);
+  const RangeWalk w = range_walk(p0c, inc);
   // a contributing run must end before the keyhole window
   const float flat_lim = fminf(kw0, tend);
   // a repeated alpha is the cheap hint of a constant brick
@@ -277,7 +316,7 @@ __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMa
         if (TERM && acc <= stop_at) break;
         // each further sample of a contributing run steps 1 (sa = sb = 0)
         if (FV::kFlatRuns && runs && repeat && z == 0.0f) {
-          if (flat_run(a, q, p0c, inc, w, cs, ci, alpha, t, t >= kw1 ? tend : flat_lim, acc, stop_at)) break;
+          if (flat_run<TERM>(a, q, w, cs, ci, alpha, t, t >= kw1 ? tend : flat_lim, 1.0f, 1.0f, acc, stop_at)) break;
         }
       } else {
         if (!PRECISE) {
@@ -289,9 +328,9 @@ __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMa
         t += 1.0f + z;
         // each further non-contributing sample steps 2 and leaves sb = 1
         if (runs) {
-          const int m = empty_run(a, q, p0c, inc, w, cs, ci, t, tend, 2.0f);
-          if (m > 0) {
-            t += 2.0f * (float)m;
+          const float m = empty_run(a, q, w, cs, ci, t, tend, 0.5f);
+          if (m > 0.0f) {
+            t += 2.0f * m;
             z = 1.0f;
           }
         }
@@ -304,20 +343,152 @@ __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMa
         if (VG) visit(q, ts, alpha, gr);
         if (TERM && acc <= stop_at) break;
         if (FV::kFlatRuns && runs && repeat) {
-          if (flat_run(a, q, p0c, inc, w, cs, ci, alpha, t, t >= kw1 ? tend : flat_lim, acc, stop_at)) break;
+          if (flat_run<TERM>(a, q, w, cs, ci, alpha, t, t >= kw1 ? tend : flat_lim, 1.0f, 1.0f, acc, stop_at)) break;
         }
       } else if (runs) {
-        t += (float)empty_run(a, q, p0c, inc, w, cs, ci, t, tend, 1.0f);
+        t += empty_run(a, q, w, cs, ci, t, tend, 1.0f);
       }
     }
   }
-  const float L = (float)acc;
-  if (ref_mode) {
-    const float o = 256.0f - expf(L);
-    return o < 0.0f ? 0.0f : o;
+  return drr_value(a, (float)acc);
+}
+
+// The same line integral with 2^ls lanes of a wave on one ray, for launches
+// with too few rays to fill the device (a wave then waits on one chain of
+// dependent samples: 128^2 rays of ~100 samples took 63 us, 0.5 us a sample,
+// with one wave on every fourth SIMD).  Lane s of the ray's 2^ls takes
+// samples s, s + 2^ls, ...; the f64 partial sums are added at the end.
+// Precise march, no termination (both tests are the caller's).
+//
+// The skip rule makes which samples count depend on the ones before, so its
+// lanes take a chunk of samples at once, speculatively, and keep what the
+// serial march would have: it runs either sample by sample (each one counts,
+// until the first empty one at u: the next looked at is u + 2) or two by two
+// (until the first contributing one at u: the march steps back to u - 1,
+// which counts if it contributes, and goes on sample by sample from u).
+// Either way the chunk's first change of run, found in the ballot of the
+// samples' signs, says where the next chunk starts.
+template <typename CV, bool SKIP, bool VG = false, typename F = NoVisit>
+__device__ __forceinline__ float drr_march_lanes(CV vol, const VolGeom& g, const DrrMarchArgs& a, const Ray& r, int x,
+                                                 int y, int ls, F&& visit = F()) {
+  const int S = 1 << ls, lane = (int)(threadIdx.x & 63u);
+  const int s = lane & (S - 1), first = lane & ~(S - 1);
+  const float j = ray_offset(a.jitter, x, y);
+  const V3<float> p{r.start.x + j * r.inc.x, r.start.y + j * r.inc.y, r.start.z + j * r.inc.z};
+  const V3<float> inc = r.inc, p0c = cell_coord(p);
+  int kst = step_count(r.num_steps - j);
+  if (!samples_in_cells(g, p0c, inc, kst)) kst = 0;
+  const float ds = ray_length(g, inc);
+  const float ci = a.intercept * -ds;
+  const float cs = a.slope * -ds;
+  const int es = kst - (int)ceilf(r.exclude_start);
+  const int ee = kst - (int)floorf(r.exclude_end);
+  const float tend = (float)kst, kw0 = (float)(kst - es), kw1 = (float)(kst - ee);
+  const float fS = (float)S, fs = (float)s;
+  double acc = 0.0;
+  V3<float> gr{0.0f, 0.0f, 0.0f};
+  auto sample = [&](float t) {
+    const V3<float> q = sample_pos<true>(p, p0c, inc, t);
+    return fmaf(cs, VG ? trilinear_vg<false>(vol, g, q.x, q.y, q.z, gr) : trilinear<false>(vol, g, q.x, q.y, q.z), ci);
+  };
+  const bool runs = a.ranges != nullptr;
+  const RangeWalk w = range_walk(p0c, inc);
+  const float flat_lim = fminf(kw0, tend);  // a contributing run ends before the keyhole window
+  if (SKIP) {
+    const uint32_t all = (1u << S) - 1u;
+    float t = 0.0f;        // the chunk's first sample, the same in the ray's lanes
+    bool two = false;      // running two by two
+    uint32_t stepped = 0;  // 1: the chunk's first sample is a step back
+    while (t < tend) {
+      const float ts = fmaf(fs, two ? 2.0f : 1.0f, t);
+      const bool in = ts < tend;
+      const float tq = in ? ts : t;
+      const float alpha = sample(tq);
+      const bool c = in && alpha < 0.0f && !(tq >= kw0 && tq < kw1);
+      const uint32_t bits = (uint32_t)(__ballot(c) >> first) & all;
+      // two by two: samples before the first contributing one; one by one:
+      // before the first empty one (a step back goes on from its successor)
+      const int run = __ffs((two ? bits : ~(bits | stepped)) | (1u << S)) - 1;
+      const bool whole = run == S;
+      if (!two && s < run && c) {
+        acc += (double)alpha;
+        if (VG) visit(V3<float>{}, tq, alpha, gr);
+      }
+      t += two ? (whole ? 2.0f * fS : (float)(2 * run - 1)) : (whole ? fS : (float)(run + 2));
+      stepped = (two && !whole) ? 1u : 0u;
+      // a chunk that ended in its run: the run may go on through q's region
+      // (samples one by one only when all alphas of the chunk were equal)
+      if (runs && whole && t < tend) {
+        const bool flat = (((__ballot(alpha == __shfl(alpha, first, 64)) >> first) & all) == all);
+        if (two || flat) {
+          const V3<float> q = sample_pos<true>(p, p0c, inc, t);
+          if (two) {
+            t = fmaf(empty_run(a, q, w, cs, ci, t, tend, 0.5f), 2.0f, t);
+          } else {
+            double add = 0.0;
+            flat_run<false>(a, q, w, cs, ci, alpha, t, t >= kw1 ? tend : flat_lim, 1.0f, 1.0f, add, 0.0);
+            if (s == 0) acc += add;
+          }
+        }
+      }
+      two = two == whole;
+    }
+  } else {
+    const float rS = 1.0f / fS;
+    float alpha_prev = __builtin_nanf("");
+    float t = fs;
+    while (t < tend) {
+      const V3<float> q = sample_pos<true>(p, p0c, inc, t);
+      const float alpha = sample(t);
+      const bool repeat = alpha == alpha_prev;
+      alpha_prev = alpha;
+      const float ts = t;
+      t += fS;
+      if (alpha < 0.0f && !(ts >= kw0 && ts < kw1)) {
+        acc += (double)alpha;
+        if (VG) visit(V3<float>{}, ts, alpha, gr);
+        if (runs && repeat) flat_run<false>(a, q, w, cs, ci, alpha, t, t >= kw1 ? tend : flat_lim, fS, rS, acc, 0.0);
+      } else if (runs) {
+        t = fmaf(empty_run(a, q, w, cs, ci, t, tend, rS), fS, t);
+      }
+    }
   }
-  if (a.output == RVK_DRR_F32_EXP_NEG_L) return expf(L);
-  return -L;
+  for (int o = 1; o < S; o <<= 1) acc += __shfl_xor(acc, o, 64);
+  return drr_value(a, (float)((a.output == RVK_DRR_RGBA8_REF ? (double)logf(256.0f * a.offset) : 0.0) + acc));
+}
+
+// Pixel of index i (0..255) of a 16x16 tile in Morton order: any aligned
+// power-of-two run of indices is a compact block.
+__device__ __forceinline__ void morton_pixel(int i, int& x, int& y) {
+  x = (i & 1) | ((i >> 1) & 2) | ((i >> 2) & 4) | ((i >> 3) & 8);
+  y = ((i >> 1) & 1) | ((i >> 2) & 2) | ((i >> 3) & 4) | ((i >> 4) & 8);
+}
+
+// Pixel of a lane when 2^ls lanes share a ray: workgroup `blk` takes part
+// blk mod 2^ls of 16x16 tile blk >> ls (in the launch's super-tile order).
+__device__ __forceinline__ void lanes_pixel(int blk, int stiles_x, int ls, int& x, int& y) {
+  int tx, ty;
+  tile_origin(blk >> ls, stiles_x, tx, ty);
+  morton_pixel(((blk & ((1 << ls) - 1)) << (8 - ls)) | ((int)threadIdx.x >> ls), x, y);
+  x += tx;
+  y += ty;
+}
+
+// The DRR caster's pixel: exp(-L) or L, or the tinted RGBA8
+// (V/...DRR...cuh:163-166).
+__device__ __forceinline__ void drr_store(const DrrArgs& a, int x, int y, float v) {
+  const long idx = (long)y * a.v.W + x;
+  if (a.m.output == RVK_DRR_RGBA8_REF) {
+    const float tw = (float)(a.tint >> 24);
+    const float q = tw / (tw + v);
+    const uint32_t A = to_u8(tw + (1.0f - tw / 255.0f) * v);
+    const uint32_t R = to_u8(q * (float)(a.tint & 255u));
+    const uint32_t G = to_u8(q * (float)((a.tint >> 8) & 255u));
+    const uint32_t B = to_u8(q * (float)((a.tint >> 16) & 255u));
+    ((uint32_t*)a.out)[idx] = R | (G << 8) | (B << 16) | (A << 24);
+  } else {
+    ((float*)a.out)[idx] = v;
+  }
 }
 
 }  // namespace rvk

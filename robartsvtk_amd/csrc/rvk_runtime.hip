@@ -374,6 +374,22 @@ __global__ __launch_bounds__(256) void frame_stats_kernel(const VT* __restrict__
   }
 }
 
+// Ranges of the groups of 4^3 range bricks, one wave per group.  (Groups of
+// constant bricks of one value are constant; a brick's widened bounds stay.)
+__global__ __launch_bounds__(64) void range_groups_kernel(const float2* __restrict__ ranges, int rbx, int rby, int rbz,
+                                                          int gx, int gy, float2* __restrict__ groups) {
+  const int g = blockIdx.x, l = threadIdx.x;
+  const int bx = min((g % gx) * 4 + (l & 3), rbx - 1), by = min((g / gx % gy) * 4 + ((l >> 2) & 3), rby - 1);
+  const int bz = min(g / (gx * gy) * 4 + (l >> 4), rbz - 1);
+  float2 r = ranges[((size_t)bz * rby + by) * rbx + bx];
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    r.x = fminf(r.x, __shfl_xor(r.x, o, 64));
+    r.y = fmaxf(r.y, __shfl_xor(r.y, o, 64));
+  }
+  if (l == 0) groups[g] = r;
+}
+
 // Binary16 cells -> difference cells: each x-pair's base (and, for
 // HalfPair cells, its difference) becomes the 16-bit integer it holds
 // (exact); an int16 difference stays.
@@ -409,6 +425,8 @@ static int launch_stats(rvk_volume* v, int frame, const void* dsrc) {
   if (sizeof(VT) == 2) hipLaunchKernelGGL(stats_init_kernel, dim3(1), dim3(kStatSlots), 0, s, stats);
   hipLaunchKernelGGL((frame_stats_kernel<VT>), dim3((tasks + 3) / 4), dim3(256), 0, s, (const VT*)dsrc, v->dims[0],
                      v->dims[1], v->dims[2], v->nrb[0], v->nrb[1], v->nrb[2], v->ranges[frame], stats);
+  hipLaunchKernelGGL(range_groups_kernel, dim3((unsigned)v->n_range_groups()), dim3(64), 0, s, v->ranges[frame],
+                     v->nrb[0], v->nrb[1], v->nrb[2], v->nrg(0), v->nrg(1), v->range_groups(frame));
   RVK_HIP(hipGetLastError());
   return RVK_OK;
 }
@@ -416,7 +434,7 @@ static int launch_stats(rvk_volume* v, int frame, const void* dsrc) {
 static int frame_stats(rvk_volume* v, int frame, const void* dsrc, int& lo, int& hi, bool& odd_diff) {
   if (!v->ranges[frame]) {
     void* q = nullptr;
-    RVK_HIP(hipMalloc(&q, sizeof(float2) * v->n_range_bricks() + kStatBytes));
+    RVK_HIP(hipMalloc(&q, sizeof(float2) * (v->n_range_bricks() + v->n_range_groups()) + kStatBytes));
     v->ranges[frame] = (float2*)q;
   }
   int rc = RVK_OK;

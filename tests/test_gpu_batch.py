@@ -774,3 +774,73 @@ def test_pose_gradient_at_h_1e3_on_a_smooth_phantom(gpu_ctx):
         assert er <= 1e-3 and et <= 1e-3, (v, er, et)
     plan.close()
     vol.close()
+
+
+@pytest.mark.parametrize("n_views,w,h", [(1, 9, 7), (1, 128, 96), (2, 200, 100), (2, 200, 180), (4, 330, 310),
+                                         (6, 340, 350)])
+@pytest.mark.parametrize("dtype,skip,keyhole", [("f32", 0, False), ("f32", 1, True), ("i16", 1, False),
+                                                ("i16", 0, True), ("u8", 0, False)])
+def test_several_lanes_per_ray_march_as_one(gpu_ctx, n_views, w, h, dtype, skip, keyhole):
+    """The default schedule puts 2 to 16 lanes on a ray where a launch has few
+    rays (here each count, and its edges); the persistent schedule has one.
+    The same samples count, in another order: f64 sums of n terms differ by
+    n 2^-53 relative, so L differs by the f32 rounding, one ulp; the per-ray
+    f32 gradient sums of n <= 400 terms and their per-view sums differ by less
+    than 1e-4 of the largest gradient.  Single views take the single-view
+    schedule, against the same plan."""
+    import torch
+    n, spacing = (70, 66, 61), (1.0, 1.1, 1.2)
+    rng = np.random.default_rng(w)
+    z, y, x = np.meshgrid(*[np.linspace(-1, 1, k) for k in n[::-1]], indexing="ij")
+    body = (x * x + y * y + z * z) < 0.5
+    vol = np.where(body, rng.uniform(0.0, 200.0, n[::-1]), 0.0)
+    vol[20:36, 20:36, 20:36] = 150.0  # a constant block, and empty space around the body
+    vol[40:44, 30:34, 5:60] = 0.0
+    vol = np.rint(vol).astype({"f32": np.float32, "i16": np.int16, "u8": np.uint8}[dtype])
+    c = configs.volume_center(n, spacing)
+    views, dms = [], []
+    for i in range(n_views):
+        cam = configs.drr_camera(c, 0.4 + 0.9 * i, h, sod=300.0, sid=600.0, fov=200.0, half_extent=75.0)
+        v, dm = abi.posed_view(cam, [0.05 * i, 0.1, -0.08, 1.0, -2.0, 0.5], c, w, h, spacing=spacing,
+                               with_derivatives=True)
+        if keyhole:
+            v.n_keyhole_planes = 2
+            v.keyhole_planes[:8] = [1.0, 0.0, 0.0, -25.0, -1.0, 0.0, 0.0, 45.0]
+        views.append(v)
+        dms.append(dm)
+    march = configs.march_params({"step_scale": 0.4, "term_T": 0.0, "jitter": 1, "skip_rule": skip})
+    drr = configs.drr_params({"intercept": -1e-5, "slope": 1e-4, "offset": 1.0, "output": abi.DRR_F32_L,
+                              "ref_termination": 0})
+    vh = H.gpu_volume(gpu_ctx, vol, spacing)
+    plan = abi.DrrPlan(gpu_ctx, vh, views, march, drr, dview=np.stack(dms))
+    tgt = torch.from_numpy(rng.uniform(0, 1, plan.total).astype(np.float32)).cuda()
+    got = {}
+    for sched in (abi.SCHED_GRID, abi.SCHED_PERSISTENT):
+        plan.set_schedule(sched)
+        out, reg = (torch.full((plan.total,), float("nan"), device="cuda") for _ in range(2))
+        loss, grad = torch.empty(n_views, device="cuda"), torch.empty(6 * n_views, device="cuda")
+        plan.render(out)
+        plan.register(reg, tgt, loss, grad)
+        torch.cuda.synchronize()
+        got[sched] = [t.cpu().numpy() for t in (out, reg, grad)]
+    one, many = got[abi.SCHED_PERSISTENT], got[abi.SCHED_GRID]
+    assert one[0].max() > 0.1 and (one[0] == 0.0).any()
+    ulp = 2.0 ** -23 * np.abs(one[0])
+    assert np.all(np.abs(many[0] - one[0]) <= ulp) and np.all(np.abs(many[1] - one[1]) <= ulp)
+    g1, g2 = one[2].reshape(-1, 6), many[2].reshape(-1, 6)
+    assert np.all(np.abs(g1 - g2) <= 1e-4 * np.abs(g1).max())
+    # the adjoint (one lane) against the register step's own gradient of the same loss
+    dldi = torch.empty(plan.total, device="cuda")
+    img = torch.from_numpy(one[0]).cuda()
+    bwd = torch.empty(6 * n_views, device="cuda")
+    plan.ncc(img, tgt, loss, dldi)
+    plan.backward(img, dldi, grad_pose=bwd)
+    single = torch.full((h, w), float("nan"), device="cuda")
+    for i, v in enumerate(views):
+        abi.render_drr(gpu_ctx, vh, v, march, drr, single)
+        torch.cuda.synchronize()
+        s, o = single.cpu().numpy().ravel(), one[0][plan.offsets[i]:plan.offsets[i + 1]]
+        assert np.all(np.abs(s - o) <= 2.0 ** -23 * np.abs(o)), i
+    assert np.all(np.abs(bwd.cpu().numpy().reshape(-1, 6) - g1) <= 1e-4 * np.abs(g1).max())
+    plan.close()
+    vh.close()
