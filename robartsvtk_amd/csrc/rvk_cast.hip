@@ -14,6 +14,7 @@
 #include <cmath>
 #include <mutex>
 
+#include "rvk_cast.h"
 #include "rvk_lanes.h"
 
 namespace rvk {
@@ -39,22 +40,6 @@ __global__ __launch_bounds__(256) void drr_kernel(DrrArgs a) {
 
 // ===========================================================================
 // 1D transfer function
-struct Cast1dArgs {
-  VolGeom g;
-  ViewGeom v;
-  float step_len, term_T;
-  int jitter;
-  int n;
-  rvk_tf1d_params p;
-  const float* tables;
-  const void* vol;
-  uint32_t* out;
-  float* depth;
-  float* min_depth;
-  float* max_depth;
-  int tiles_x;
-};
-
 // V/...1D...cuh:27-172.  GRAD=false is taken only when the gradient cannot
 // change the result: diffuse = specular = 0, specular power >= 0 and no
 // gradient-opacity table (non-finite multiplier); then shadeD = ambient and
@@ -170,32 +155,6 @@ __global__ __launch_bounds__(256) void cast1d_kernel(Cast1dArgs a) {
 
 // ===========================================================================
 // 2D transfer function
-struct Cast2dArgs {
-  VolGeom g;
-  ViewGeom v;
-  float step_len, term_T;
-  int jitter;
-  int n;
-  rvk_tf2d_params p;
-  const Tf2dCell* cells;
-  const Tf2dCell* kcells;
-  const float4* lit;     // the cells lit with a Phong-Lambert factor of 1 (GMAG)
-  const float4* klit;
-  const uint32_t* occ;   // opacity bitmaps staged in LDS, or NULL
-  const uint32_t* kocc;
-  int occ_words;
-  const uint32_t* col;   // column bitmaps (TF, then keyhole TF), staged in LDS
-  int col_words;
-  const void* vol;
-  const uint8_t* gradmag;
-  float gradmag_scale;
-  uint32_t* out;
-  float* depth;
-  float* min_depth;
-  float* max_depth;
-  int tiles_x;
-};
-
 // V/...2D...cuh:30-351.  DUAL selects the keyhole-TF variant (WithDual).
 // GMAG reads |grad| from the precomputed u8 volume instead of 6 extra gathers;
 // without a direction the Phong-Lambert factor is taken as 1, so a table
@@ -434,12 +393,7 @@ int rvk_render_drr(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk_vie
            ((uint32_t)drr->tint[3] << 24);
   a.vol = vol->frames[frame];
   a.out = out;
-  a.m.ranges = vol->ranges[frame];
-  a.m.rbx = vol->nrb[0];
-  a.m.rby = vol->nrb[1];
-  a.m.groups = vol->range_groups(frame);
-  a.m.rgx = vol->nrg(0);
-  a.m.rgy = vol->nrg(1);
+  set_ranges(a.m, vol, frame);
   const int nblk = launch_grid(view, a.tiles_x);
   const DrrSchedule sch = drr_schedule(vol, (long long)view->width * view->height, a.step_len);
   const bool runs = march->precise && !drr->ref_termination;
@@ -500,6 +454,8 @@ int rvk_render_1d(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk_tf1d
   const bool grad = !(tf->p.diffuse == 0.0f && tf->p.specular == 0.0f && tf->p.specular_power >= 0.0f &&
                       !std::isfinite(tf->p.gradient_multiplier));
   const bool skip = march->skip_rule != 0, pr = march->precise != 0;
+  set_ranges(a.m, vol, frame);
+  if (quad_ok(view, march)) return launch_quad_1d(a, vol, frame, skip, grad, lds, nblk, ctx->stream);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
 #define RVK_L1D(S, G, P) \
@@ -558,6 +514,8 @@ int rvk_render_2d(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk_tf2d
   const int nblk = launch_grid(view, a.tiles_x);
   const bool skip = march->skip_rule != 0, dual = tf->kcells != nullptr, gm = use_gradmag != 0;
   const bool pr = march->precise != 0;
+  // without keyhole planes no sample takes the keyhole TF
+  if (quad_ok(view, march)) return launch_quad_2d(a, vol, frame, skip, gm, lds, nblk, ctx->stream);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
 #define RVK_L2D(S, D, G)                                                                              \

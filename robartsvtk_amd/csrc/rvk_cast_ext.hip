@@ -12,35 +12,12 @@
 #include <cmath>
 #include <type_traits>
 
-#include "rvk_internal.h"
-#include "rvk_march.h"
+#include "rvk_cast.h"
 
 namespace rvk {
 
 // ===========================================================================
 // 2D TF with in/ex logic
-struct InExArgs {
-  VolGeom g;
-  ViewGeom v;
-  float step_len, term_T;
-  int jitter;
-  int n;
-  int black_keyhole;
-  rvk_tf2d_params p;
-  const Tf2dCell* cells;
-  const uint8_t* flags;  // per cell: bit 0 composites, bit 1 excludes
-  const uint32_t* occ;   // the same as two bitmaps (occ_words each), or NULL
-  int occ_words;
-  const uint32_t* col;   // column bitmap of bit 0 (col_words), staged in LDS
-  int col_words;
-  const void* vol;
-  uint32_t* out;
-  float* depth;
-  float* min_depth;
-  float* max_depth;
-  int tiles_x;
-};
-
 // V/...InExLogic...cuh:24-179.  Against the 2D caster: the step count is
 // floor(numSteps) (the ray offset moves the start only), a sample composites
 // when inEx > 0 or alpha > 0, the first composited sample outside the
@@ -158,37 +135,6 @@ __global__ __launch_bounds__(256) void inex_kernel(InExArgs a) {
 
 // ===========================================================================
 // Dual-image caster
-struct DualArgs {
-  VolGeom g;
-  ViewGeom v;
-  float step_len, term_T;
-  int jitter;
-  int n;
-  rvk_dual_params p;
-  const Tf2dCell* cells;
-  const Tf2dCell* kcells;
-  const uint32_t* occ;  // opacity bitmaps staged in LDS, or NULL
-  const uint32_t* kocc;
-  int occ_words;
-  const uint32_t* col;  // column bitmaps (TF, then keyhole TF), staged in LDS
-  int col_words;
-  const void* vol1;
-  const void* vol2;
-  uint32_t* out;
-  float* depth;
-  float* min_depth;
-  float* max_depth;
-  int tiles_x;
-};
-
-// Ray samples of the dual caster: floor(numSteps) less the ray offset,
-// truncated (V/...DualImage...cuh:66-67 store an int minus a float back in an
-// int); rays the 2D caster would not march march nothing here either.
-__device__ __forceinline__ int dual_step_count(float num_steps, float j) {
-  if (!(num_steps > 0.0f && num_steps < 16777216.0f)) return 0;
-  return (int)((float)(int)floorf(num_steps) - j);
-}
-
 // V/...DualImage...cuh:33-380.  The table is indexed by the two components
 // (component 1 the column, component 2 the row); shading uses the gradient of
 // component 1.  KEYTF selects the keyhole-TF variant; without it the march
@@ -349,6 +295,9 @@ int rvk_render_2d_inex(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk
   a.max_depth = aux ? aux->max_depth : nullptr;
   const int nblk = launch_grid(view, a.tiles_x);
   const bool skip = march->skip_rule != 0, pr = march->precise != 0;
+  set_ranges(a.m, vol, frame);
+  // (its keyhole window is a test, not a jump)
+  if (pr && march->term_T <= 1.0f) return launch_quad_inex(a, vol, frame, skip, lds, nblk, ctx->stream);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
 #define RVK_LIE(S, P) hipLaunchKernelGGL((inex_kernel<CV, S, P>), dim3(nblk), dim3(256), lds, ctx->stream, a)
@@ -406,6 +355,8 @@ int rvk_render_dual(rvk_ctx* ctx, const rvk_volume* vol1, const rvk_volume* vol2
   rc = frame_drop_half(vol1, frame, ctx->stream);
   if (!rc) rc = frame_drop_half(vol2, frame, ctx->stream);
   if (rc) return rc;
+  set_ranges(a.m, vol1, frame);
+  if (quad_ok(view, march)) return launch_quad_dual(a, vol1, vol2, frame, skip, lds, nblk, ctx->stream);
   return dispatch_frame<false>(vol1, frame, [&](auto tag1) {
     using CV = decltype(tag1);
     return dispatch_frame<false>(vol2, frame, [&](auto tag2) {

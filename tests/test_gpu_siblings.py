@@ -270,3 +270,92 @@ def test_sibling_errors(gpu_ctx):
     torch.cuda.synchronize()
     for o in (t, h1, small, other):
         o.close()
+
+
+# ---------------------------------------------------------------------------
+# Four lanes per ray against one
+def _no_window(view):
+    """A keyhole plane that leaves every ray outside: the window is empty, but
+    the view takes the casters that march one lane per ray."""
+    v = abi.View.from_buffer_copy(view)
+    v.n_keyhole_planes = 1
+    v.keyhole_planes[:4] = [1.0, 0.0, 0.0, -1e6]
+    return v
+
+
+@pytest.mark.parametrize("W,h", [(1, 1), (7, 5), (37, 18), (130, 67)])
+@pytest.mark.parametrize("dtype", ["u8", "i16", "u16", "f32"])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_four_lanes_composite_as_one(gpu_ctx, W, h, dtype, skip):
+    """1D (with and without gradients), 2D (gradient magnitude, gradients; a
+    table with and without its bitmap in LDS) and dual renders, and their
+    depth outputs, are the same to the bit as the one-lane casters': runs of
+    empty and constant bricks, noise across the transfer function's edges
+    (the skip rule's step back), early termination and none."""
+    import torch
+    dims, spacing = (53, 41, 46), (1.0, 1.2, 0.9)
+    rng = np.random.default_rng(W * 7 + skip)
+    z, y, x = np.meshgrid(*[np.linspace(-1, 1, k) for k in dims[::-1]], indexing="ij")
+    body = x * x + y * y + z * z < 0.6
+    base = np.where(body, 90.0 + 60.0 * x + rng.uniform(-25, 25, dims[::-1]), 10.0)
+    base[8:24, 8:24, 8:24] = 140.0
+    vol = np.rint(np.clip(base, 0, 255)).astype({"u8": np.uint8, "i16": np.int16, "u16": np.uint16,
+                                                 "f32": np.float32}[dtype])
+    c = configs.volume_center(dims, spacing)
+    cam = abi.camera(c + np.array([70.0, 90.0, 40.0]), c, (0, 0, 1), 30.0, (50.0, 200.0))
+    view = abi.compute_view(cam, W, h, spacing=spacing)
+    vh, vh2 = (H.gpu_volume(gpu_ctx, a, spacing) for a in (vol, vol[::-1].copy()))
+    vh.compute_gradmag(0, 60.0)
+    ramp = np.clip((np.arange(300) - 100.0) / 400.0, 0.0, 1.0).astype(np.float32)
+    rgb = rng.uniform(0, 1, (300, 3)).astype(np.float32)
+    tfs = [abi.TF1D(gpu_ctx, ramp, rgb, abi.Tf1dParams(0.0, 1 / 255.0, 0.0, float("inf"), 1.0, 0.0, 0.0, 1.0)),
+           abi.TF1D(gpu_ctx, ramp, rgb, abi.Tf1dParams(0.0, 1 / 255.0, 0.0, 1 / 60.0, 0.4, 0.6, 0.3, 8.0),
+                    galpha=np.linspace(0.2, 1, 300))]
+    tables = []
+    for n in (64, 300):
+        t = configs.tf2d_bumps(5, n)
+        t["alpha"] = np.where(np.arange(n)[None, :] > 0.3 * n, 0.3 * t["alpha"] + 0.02, 0.0)
+        t["diffuse"] = np.full((n, n), 0.6, np.float32)
+        t["specular"] = np.full((n, n), 0.3, np.float32)
+        tables.append(abi.TF2D(gpu_ctx, t, configs.tf2d_params(configs.tf2d_params_for(0.0, 255.0, 0.0, 60.0))))
+    dual = abi.DualParams(0.0, 1 / 255.0, 0.0, 1 / 255.0)
+    for term in (0.0, 0.05, 1.0):
+        march = configs.march_params({"step_scale": 0.7, "term_T": term, "jitter": 1, "skip_rule": skip})
+        calls = [lambda v, o, a, tf=tf: abi.render_1d(gpu_ctx, vh, tf, v, march, o, a) for tf in tfs]
+        for tf in tables:
+            calls += [lambda v, o, a, tf=tf, gm=gm: abi.render_2d(gpu_ctx, vh, tf, v, march, o, gm, a)
+                      for gm in (True, False)]
+            calls.append(lambda v, o, a, tf=tf: abi.render_dual(gpu_ctx, vh, vh2, tf, dual, v, march, o, a))
+        for i, call in enumerate(calls):
+            got = []
+            for v in (view, _no_window(view)):
+                out = torch.full((h, W, 4), 77, dtype=torch.uint8, device="cuda")
+                d = [torch.full((h, W), float("nan"), device="cuda") for _ in range(3)]
+                call(v, out, abi.AuxOut(*[b.data_ptr() for b in d]))
+                torch.cuda.synchronize()
+                got.append([b.cpu().numpy() for b in (out, *d)])
+            for p, q in zip(*got):
+                assert np.array_equal(p, q, equal_nan=p.dtype.kind == "f"), (term, i, int((p != q).sum()))
+            assert min(W, h) < 16 or got[0][0].any()
+    for handle in (*tfs, *tables, vh, vh2):
+        handle.close()
+
+
+@pytest.mark.parametrize("black,key,n", [(False, False, 64), (True, True, 64), (False, True, 300)])
+@pytest.mark.parametrize("width,height", [(7, 5), (66, 43)])
+def test_inex_four_lanes_against_the_oracle(gpu_ctx, black, key, n, width, height):
+    """The in/ex caster, whose keyhole window the four-lane march tests too,
+    against the FP32 oracle: the same operations but for log2f and powf, so
+    RGBA8 within 1 LSB on 99.9 % of pixels, as elsewhere in this file."""
+    s = configs.scene_c3(scale=0.125)
+    view = abi.compute_view(s.extra["camera"], width, height, spacing=s.spacing)
+    if key:
+        _keyhole(view, s.volume.shape[0])
+    tables = configs.tf2d_bumps(3, n)
+    tf, inex = _inex_tf(tables, s.tf2d["params"])
+    march = dict(s.march, skip_rule=1, precise=1, step_scale=0.7)
+    g, gd = H.gpu_2d_inex(gpu_ctx, H.gpu_volume(gpu_ctx, s.volume, s.spacing), tf, inex, black, view, march, True)
+    o, _, od = orc.cast2d_inex(s.volume, s.spacing, tf, inex, black, configs.view_dict(view), march, "f32")
+    f, m = H.lsb_stats(g, o)
+    assert f >= 0.999, (f, m)
+    assert np.mean(gd[0] == np.asarray(od).reshape(gd[0].shape)) >= 0.999
