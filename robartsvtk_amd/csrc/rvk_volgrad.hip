@@ -16,14 +16,25 @@
 // from layer to layer, held in LDS; at the slab's end the sums go to the
 // volume's by global atomics.  So each sample is gathered once, in the order
 // of the rays, and passes over empty bricks as the forward does.  Bound by
-// VALU issue.
+// VALU issue (about 95 instructions a sample) and the wait for the gather.
+// (One workgroup per 8^3-voxel brick, re-marching the stretch of every ray
+// that meets it, gathered each sample 1.4 times over and kept 55 % of its
+// lanes: 7858 us and a ray record pass for the 256^3 case below.)
 #include "rvk_volgrad.h"
+
+#include <type_traits>
 
 namespace rvk {
 
 constexpr int kVgNonFinite = 1 << 30;
-constexpr int kVgCap = 2560;       // LDS sums: 20 KiB, 7 workgroups per CU
-constexpr int kVgMaxLayers = 24;   // layers of cells in a slab
+// Sums a workgroup holds (25 KiB: 6 workgroups per CU, as its registers allow)
+// and the most layers of cells in a slab.  Volume gradient, us, with room for
+// 1536 / 2560 / 3200 / 3840 / 5120 sums: 256^3 16 x 512^2 (a tile spans 8 voxels)
+// 4180 / 4192 / 4179 / 4552 / 6273, 200^3 8 x 400^2 757 / 727 / 731 / 784 / 1028,
+// 128x128x100 4 x 200^2 (20 voxels) 661 / 422 / 354 / 330 / 310.  Registers for 5, 7
+// or 8 workgroups per CU 4572 / 4373 / 5168; slabs of 24 layers 4358, of 12 4192.
+constexpr int kVgCap = 3200;
+constexpr int kVgMaxLayers = 8;
 
 struct VgRay {
   V3<float> p0c, inc;
@@ -139,7 +150,7 @@ __device__ __forceinline__ void vg_global_add(const VolGradArgs& a, int x, int y
 __device__ __forceinline__ float vg_axis(const V3<float>& v, int d) { return d == 0 ? v.x : d == 1 ? v.y : v.z; }
 
 template <typename CV>
-__global__ __launch_bounds__(256) void vg_scatter_kernel(VolGradArgs a) {
+__global__ __launch_bounds__(256, 6) void vg_scatter_kernel(VolGradArgs a) {
   __shared__ unsigned long long s_acc[kVgCap];
   __shared__ int s_base[kVgMaxLayers + 1], s_off1[kVgMaxLayers + 1], s_off2[kVgMaxLayers + 1];
   __shared__ float s_red[2][4][5];
@@ -185,7 +196,7 @@ __global__ __launch_bounds__(256) void vg_scatter_kernel(VolGradArgs a) {
   // whether sample t counts (its alpha, as the forward has it)
   auto counts = [&](float t, const V3<float>& q) {
     // samples in the keyhole window are not accumulated by the forward
-    if (t >= r.kw0 && t < r.kw1) return false;
+    if (bv.v.n_key && t >= r.kw0 && t < r.kw1) return false;
     return fmaf(r.cs, trilinear<false>(vol, g, q.x, q.y, q.z), r.ci) < 0.0f;
   };
   auto direct = [&](float t) {
@@ -211,6 +222,36 @@ __global__ __launch_bounds__(256) void vg_scatter_kernel(VolGradArgs a) {
   auto layer = [&](float tt) {
     const int c = (int)fmaf(tt, id, pd);
     return down ? -c : c;
+  };
+  // The ray's next cnt samples into the box, whose rows are w1 long (axis d1
+  // fastest: the corners of a sample then are four addresses and their
+  // successors).  Each lane starts at its own sample (3 x its lane) and wraps
+  // round: in step, a wave's rays would add to the same voxels in the same
+  // instructions (LDS address conflicts).
+  auto scatter = [&](auto axis, int cnt, int L0, int w1) {
+    constexpr int D = decltype(axis)::value;
+    const int top = kVgCap - 2 - w1;
+    int mm = (int)(3 * (tid & 63)) % cnt;
+    for (int i = 0; i < cnt; ++i, mm = mm + 1 == cnt ? 0 : mm + 1) {
+      const float ts = t + (float)mm;
+      const V3<float> q = at(ts);
+      if (!counts(ts, q)) continue;
+      const int cx = (int)q.x, cy = (int)q.y, cz = (int)q.z;
+      const int cd = D == 0 ? cx : D == 1 ? cy : cz, c1 = D == 0 ? cy : cx, c2 = D == 2 ? cy : cz;
+      const int j = (down ? -cd : cd) - L0;
+      // the lower corner's address in the layers of the lower and upper voxel
+      const int lat = (c1 - 1) + __mul24(c2 - 1, w1);
+      const int b0 = s_base[j], b1 = s_base[j + 1];
+      unsigned long long* const e0 = s_acc + min(max((down ? b1 : b0) + lat, 0), top);
+      unsigned long long* const e1 = s_acc + min(max((down ? b0 : b1) + lat, 0), top);
+      unsigned long long* const f0 = e0 + w1;
+      unsigned long long* const f1 = e1 + w1;
+      vg_corners(q, coef, [&](int dx, int dy, int dz, unsigned long long v) {
+        const int hd = D == 0 ? dx : D == 1 ? dy : dz, h1 = D == 0 ? dy : dx, h2 = D == 2 ? dy : dz;
+        __hip_atomic_fetch_add((hd ? (h2 ? f1 : e1) : (h2 ? f0 : e0)) + h1, v, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+      });
+    }
   };
   int ref = 0;  // the first slab's first layer; the box's shear starts there
   for (int it = 0;; ++it) {
@@ -272,14 +313,12 @@ __global__ __launch_bounds__(256) void vg_scatter_kernel(VolGradArgs a) {
     const int w2 = __builtin_amdgcn_readfirstlane((int)floorf(hi2 + sh2 + fabsf(slope2) + 1.0f + eps)) - b2 + 1;
     const bool fits = w1 <= kVgCap && w2 <= kVgCap && w1 * w2 * 2 <= kVgCap;
     const int T = fits ? min(kVgMaxLayers, kVgCap / (w1 * w2) - 1) : kVgMaxLayers;
-    // x is the fastest axis of the box, as of the volume
-    const int sd = d == 0 ? 1 : w1 * w2, s1 = d == 0 ? T + 1 : 1, s2 = d == 0 ? (T + 1) * w1 : w1;
     if (fits && tid <= T) {
       const float v = (float)(L0 + tid - ref);
       const int o1 = (int)floorf(slope1 * v), o2 = (int)floorf(slope2 * v);
       s_off1[tid] = o1;
       s_off2[tid] = o2;
-      s_base[tid] = tid * sd - (o1 + b1) * s1 - (o2 + b2) * s2;
+      s_base[tid] = tid * w1 * w2 - (o1 + b1) - (o2 + b2) * w1;
     }
     __syncthreads();
     if (active && L < L0 + T) {
@@ -290,28 +329,9 @@ __global__ __launch_bounds__(256) void vg_scatter_kernel(VolGradArgs a) {
       while (m < rest && layer(t + m) < L0 + T) m += 1.0f;
       const int cnt = (int)m;
       if (fits) {
-        // each lane starts at its own sample (3 x its lane) and wraps round:
-        // in step, a wave's rays would add to the same voxels in the same
-        // instructions (LDS address conflicts)
-        int mm = (int)(3 * (tid & 63)) % cnt;
-        for (int i = 0; i < cnt; ++i, mm = mm + 1 == cnt ? 0 : mm + 1) {
-          const float ts = t + (float)mm;
-          const V3<float> q = at(ts);
-          if (!counts(ts, q)) continue;
-          const int cx = (int)q.x, cy = (int)q.y, cz = (int)q.z;
-          const int cd = d == 0 ? cx : d == 1 ? cy : cz, c1 = d == 0 ? cy : cx, c2 = d == 2 ? cy : cz;
-          const int j = (down ? -cd : cd) - L0;
-          // lower corner's address in the layers of the lower and upper voxel
-          const int lat = (c1 - 1) * s1 + (c2 - 1) * s2;
-          const int top = kVgCap - 1 - s1 - s2;
-          const int e0 = min(max(s_base[down ? j + 1 : j] + lat, 0), top);
-          const int e1 = min(max(s_base[down ? j : j + 1] + lat, 0), top);
-          vg_corners(q, coef, [&](int dx, int dy, int dz, unsigned long long v) {
-            const int hd = d == 0 ? dx : d == 1 ? dy : dz, h1 = d == 0 ? dy : dx, h2 = d == 2 ? dy : dz;
-            __hip_atomic_fetch_add(s_acc + ((hd ? e1 : e0) + (h1 ? s1 : 0) + (h2 ? s2 : 0)), v, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-          });
-        }
+        if (d == 0) scatter(std::integral_constant<int, 0>{}, cnt, L0, w1);
+        else if (d == 1) scatter(std::integral_constant<int, 1>{}, cnt, L0, w1);
+        else scatter(std::integral_constant<int, 2>{}, cnt, L0, w1);
       } else {
         for (int i = 0; i < cnt; ++i) direct(t + (float)i);
       }
@@ -320,13 +340,18 @@ __global__ __launch_bounds__(256) void vg_scatter_kernel(VolGradArgs a) {
     __syncthreads();
     if (!fits) continue;
     const int total = (T + 1) * w1 * w2;
+    // x along the lanes: the axis of the layers when d is x
     const int r0 = d == 0 ? T + 1 : w1, r1 = d == 0 ? w1 : w2;
+    const float i0 = 1.0f / (float)r0, i1r = 1.0f / (float)r1;
     for (int e = tid; e < total; e += 256) {
-      const unsigned long long v = s_acc[e];
-      if (v == 0ull) continue;
-      s_acc[e] = 0ull;
-      const int f0 = e % r0, f1 = (e / r0) % r1, f2 = e / r0 / r1;
+      // e / r0 and so on: e < 2^12, so half a unit keeps the floats exact
+      const int g0 = (int)(((float)e + 0.5f) * i0), f0 = e - g0 * r0;
+      const int f2 = (int)(((float)g0 + 0.5f) * i1r), f1 = g0 - f2 * r1;
       const int V = d == 0 ? f0 : f2, i1 = d == 0 ? f1 : f0, i2 = d == 0 ? f2 : f1;
+      const int at_e = (V * w2 + i2) * w1 + i1;
+      const unsigned long long v = s_acc[at_e];
+      if (v == 0ull) continue;
+      s_acc[at_e] = 0ull;
       // voxel on axis d: layer L's cell holds voxels L - 1 and L, layers
       // counted down -L - 1 and -L
       const int vd = down ? -(L0 + V) : L0 + V - 1;
