@@ -326,7 +326,6 @@ __global__ __launch_bounds__(64) void pose_views_kernel(const PoseGeom* __restri
   BatchView& b = views[v];
   for (int k = 0; k < 16; ++k) b.v.m[k] = m[k];
   for (int k = 0; k < 96; ++k) b.dm[k] = dm[k];
-  pose::baked_inverse(m, b.inv);
 }
 
 struct PoseUpdateArgs {
@@ -438,8 +437,6 @@ int fill_views(rvk_drr_plan* p, const rvk_view* views, const float* dview, std::
     std::memset(&b, 0, sizeof(b));
     b.v = view_geom(&views[v]);
     if (dview) std::memcpy(b.dm, dview + 96 * (size_t)v, sizeof(b.dm));
-    // inverse of the baked matrix (Gauss-Jordan, partial pivoting)
-    pose::baked_inverse(views[v].view_to_voxels, b.inv);
     b.tiles16_x = (views[v].width + 15) / 16;
   }
   return RVK_OK;

@@ -244,10 +244,10 @@ __device__ __forceinline__ float drr_value(const DrrMarchArgs& a, float L) {
 // coordinate (c = p0 + 0.5 + t*inc in PRECISE mode); with VG the trilinear
 // gradient at c comes from the same gathers as the value (the adjoint marches
 // through this very control flow).  RUNS (precise mode only) takes the runs
-// above when the volume frame has brick ranges (a.ranges); the result is the
-// same to the bit.  Runs pay where the rays of a wave skip together (many
-// views in one launch); a single view's launch is ordered for L2 locality,
-// which runs unbalance, and marches without them.
+// above when the volume frame has brick ranges (a.ranges): the same samples
+// count, and a run's sum is rounded once instead of per sample.  Runs make the
+// tiles through empty space cheap, so their launches deal the tiles to the
+// XCDs instead of giving each a band (drr_kernel has both measured).
 template <typename CV, bool SKIP, bool PRECISE, bool VG = false, bool RUNS = false, bool KEY = true,
           bool TERM = true, typename F = NoVisit>
 __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMarchArgs& a,
