@@ -8,7 +8,7 @@ HBM.  `value` = N_samples / (seconds per render) / 1e9, with N_samples the
 plain-march ray-sample count (sum over pixels of floor(num_steps - ray
 offset)).
 
-`roofline` is the binding resource of the DRR kernel, VALU issue: its VALU
+`roofline` is the resource the DRR kernel comes closest to, VALU issue: its VALU
 instructions per launch (SQ_INSTS_VALU, committed rocprofv3 counter pass,
 profiles/kernel_counters.json) over the live kernel time, against
 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles per wave64 instruction.  The HBM
@@ -272,7 +272,7 @@ def bench_batched(scene, reps: int = 5, volume_gradient: bool = False, loop: boo
         t_vg = _time(lambda: plan.backward(out, dldi, grad_volume=gvol), max(1, reps // 2))
         assert bool(torch.isfinite(gvol).all())
         res["volume_gradient_ms"] = round(t_vg, 3)
-        res["volume_gradient_note"] = (f"rvk_drr_plan_backward(grad_volume) alone: ray records + brick-driven "
+        res["volume_gradient_note"] = (f"rvk_drr_plan_backward(grad_volume) alone: slab-wise LDS "
                                        f"fixed-point scatter over {scene.volume.size} voxels x {n} views")
     if loop:
         opt = abi.PoseOptimizer(kind=abi.OPT_ADAM, shared_pose=0, lr_rotation=0.005, lr_translation=0.5, beta1=0.9,
@@ -573,8 +573,8 @@ def main() -> int:
         c3, gpu_img = bench_compositing(scenes["c3"], max(5, args.steps // 5), min(args.warmup, 2))
         gpu["c3"] = dict(c3, image=gpu_img)
         line["casters"] = {"c1": c1, "c3": c3}
-        for k, name in (("c1", "cast1d_kernel<Cells<unsigned char,0,false>,true,false,true>"),
-                        ("c3", "cast2d_kernel<Cells<unsigned short,2,true>,true,false,true,true>")):
+        for k, name in (("c1", "quad1d_kernel<Cells<unsigned char,0,false>,true,false>"),
+                        ("c3", "quad2d_kernel<Cells<unsigned short,2,true>,true,true>")):
             cc = kernel_counters(name)
             if cc:
                 ks = line["casters"][k]["ms_per_render"] / 1e3
