@@ -20,15 +20,13 @@
 namespace rvk {
 
 // KEY = false: the view has no keyhole planes; TERM = false: no termination
-// (the accumulated sum is never compared).  The precise march without
-// termination passes over runs of empty and constant bricks: the 256^3 CT at
-// 1024^2 (skip rule) 479 -> 360 us, 1400^2 906 -> 530 us, bit for bit the
-// same images.  That needs the tiles dealt to the XCDs in runs of 8 (of a
-// super-tile of 4x4); with a band per XCD the same march takes 387 and 698 us,
-// and runs of 1, 2, 4, 16 or 32 tiles 375 / 365 / 361 / 382 / 488 us.
+// (the accumulated sum is never compared).  For the marches that neither
+// drr_lanes_kernel nor drr_ahead_kernel takes: many short rays without
+// termination, which pass over runs, the reference's positions and
+// termination.
 template <typename CV, bool SKIP, bool PRECISE, bool KEY, bool TERM>
 __global__ __launch_bounds__(256) void drr_kernel(DrrArgs a) {
-  const int tile = a.deal ? xcd_deal(blockIdx.x, kDealLog2) : xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int x, y;
   tile_pixel(tile, a.tiles_x, x, y);
   if (x >= a.v.W || y >= a.v.H) return;
@@ -400,16 +398,16 @@ int rvk_render_drr(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk_vie
   a.deal = runs && sch.deal;
   if (!sch.runs) a.m.ranges = nullptr;
   if (runs && sch.lanes) return launch_drr_lanes(a, vol, frame, march->skip_rule != 0, sch.lanes, nblk, ctx->stream);
-  const unsigned grid = a.deal ? deal_grid(nblk, kDealLog2) : (unsigned)nblk;
+  if (a.deal) return launch_drr_ahead(a, vol, frame, march->skip_rule != 0, nblk, ctx->stream);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
     const bool pr = march->precise != 0, skip = march->skip_rule != 0;
 #define RVK_LDRR2(S, P, K)                                                                                 \
   do {                                                                                                     \
     if (drr->ref_termination)                                                                              \
-      hipLaunchKernelGGL((drr_kernel<CV, S, P, K, true>), dim3(grid), dim3(256), 0, ctx->stream, a);       \
+      hipLaunchKernelGGL((drr_kernel<CV, S, P, K, true>), dim3(nblk), dim3(256), 0, ctx->stream, a);       \
     else                                                                                                   \
-      hipLaunchKernelGGL((drr_kernel<CV, S, P, K, false>), dim3(grid), dim3(256), 0, ctx->stream, a);      \
+      hipLaunchKernelGGL((drr_kernel<CV, S, P, K, false>), dim3(nblk), dim3(256), 0, ctx->stream, a);      \
   } while (0)
 #define RVK_LDRR(S, P)                                                                                     \
   do {                                                                                                     \

@@ -47,6 +47,8 @@ inline int batch_lanes(const rvk_volume* vol, long long rays, float step_len, bo
 
 // One view; nblk is the launch's count of 16x16-pixel tiles (launch_grid).
 int launch_drr_lanes(const DrrArgs& a, const rvk_volume* vol, int frame, bool skip, int ls, int nblk, hipStream_t s);
+// One view, one lane per ray, tiles dealt (rvk_ahead.hip).
+int launch_drr_ahead(const DrrArgs& a, const rvk_volume* vol, int frame, bool skip, int nblk, hipStream_t s);
 // A plan's forward (jac: with the pose Jacobians).
 int launch_batch_lanes(const BatchArgs& a, const rvk_volume* vol, int frame, bool skip, bool jac, int ls,
                        hipStream_t s);

@@ -247,7 +247,7 @@ __device__ __forceinline__ float drr_value(const DrrMarchArgs& a, float L) {
 // above when the volume frame has brick ranges (a.ranges): the same samples
 // count, and a run's sum is rounded once instead of per sample.  Runs make the
 // tiles through empty space cheap, so their launches deal the tiles to the
-// XCDs instead of giving each a band (drr_kernel has both measured).
+// XCDs instead of giving each a band (drr_ahead_kernel has both measured).
 template <typename CV, bool SKIP, bool PRECISE, bool VG = false, bool RUNS = false, bool KEY = true,
           bool TERM = true, typename F = NoVisit>
 __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMarchArgs& a,
@@ -349,6 +349,75 @@ __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMa
         t += empty_run(a, q, w, cs, ci, t, tend, 1.0f);
       }
     }
+  }
+  return drr_value(a, (float)acc);
+}
+
+// The same line integral, the sample after the next gathered along with the
+// next: where the march goes on as it did (sample by sample while samples
+// contribute, two by two while they do not) that one is the next but one, and
+// otherwise it is dropped, so the samples taken, their order and the sum are
+// drr_march's to the bit.  For single views, whose last round of waves is
+// nearly empty and waits on one gather at a time.  Precise march, no
+// termination.
+template <typename CV, bool SKIP, bool KEY>
+__device__ __forceinline__ float drr_march_ahead(CV vol, const VolGeom& g, const DrrMarchArgs& a, const Ray& r, int x,
+                                                 int y) {
+  const float j = ray_offset(a.jitter, x, y);
+  const V3<float> inc = r.inc;
+  const V3<float> p0c = cell_coord(V3<float>{r.start.x + j * inc.x, r.start.y + j * inc.y, r.start.z + j * inc.z});
+  int kst = step_count(r.num_steps - j);
+  if (!samples_in_cells(g, p0c, inc, kst)) kst = 0;
+  const float ds = ray_length(g, inc);
+  const float ci = a.intercept * -ds;
+  const float cs = a.slope * -ds;
+  const int es = kst - (int)ceilf(r.exclude_start);
+  const int ee = kst - (int)floorf(r.exclude_end);
+  const float tend = (float)kst, kw0 = (float)(kst - es), kw1 = (float)(kst - ee);
+  const float flat_lim = fminf(kw0, tend);
+  const bool runs = a.ranges != nullptr;
+  const RangeWalk w = range_walk(p0c, inc);
+  double acc = a.output == RVK_DRR_RGBA8_REF ? (double)logf(256.0f * a.offset) : 0.0;
+  float t = 0.0f;
+  float z = 0.0f;  // the skip rule's state, as in drr_march
+  float alpha_prev = __builtin_nanf("");
+  auto take = [&](const V3<float>& q, float alpha) {
+    const bool in_key = KEY && (t >= kw0 && t < kw1);
+    const bool repeat = alpha == alpha_prev;
+    alpha_prev = alpha;
+    if (alpha < 0.0f && !in_key) {
+      if (SKIP) {
+        z = __builtin_amdgcn_fmed3f(-z, -1.0f, 0.0f);
+        t += fmaf(2.0f, z, 1.0f);
+        acc += (double)fmaf(alpha, z, alpha);
+      } else {
+        t += 1.0f;
+        acc += (double)alpha;
+      }
+      if (runs && repeat && z == 0.0f)
+        flat_run<false>(a, q, w, cs, ci, alpha, t, t >= kw1 ? tend : flat_lim, 1.0f, 1.0f, acc, 0.0);
+    } else if (SKIP) {
+      z = __builtin_amdgcn_fmed3f(z + 1.0f, 0.0f, 1.0f);
+      t += 1.0f + z;
+      if (runs) {
+        const float m = empty_run(a, q, w, cs, ci, t, tend, 0.5f);
+        if (m > 0.0f) {
+          t += 2.0f * m;
+          z = 1.0f;
+        }
+      }
+    } else {
+      t += 1.0f;
+      if (runs) t += empty_run(a, q, w, cs, ci, t, tend, 1.0f);
+    }
+  };
+  while (t < tend) {
+    // the ray's end is in the cells too (samples_in_cells)
+    const float t1 = fminf(SKIP ? t + 1.0f + fmaxf(z, 0.0f) : t + 1.0f, tend);
+    const V3<float> q0 = sample_pos<true>(p0c, p0c, inc, t), q1 = sample_pos<true>(p0c, p0c, inc, t1);
+    const float v0 = trilinear<false>(vol, g, q0.x, q0.y, q0.z), v1 = trilinear<false>(vol, g, q1.x, q1.y, q1.z);
+    take(q0, fmaf(cs, v0, ci));
+    if (t == t1 && t < tend) take(q1, fmaf(cs, v1, ci));
   }
   return drr_value(a, (float)acc);
 }

@@ -846,6 +846,47 @@ def test_several_lanes_per_ray_march_as_one(gpu_ctx, n_views, w, h, dtype, skip,
     vh.close()
 
 
+@pytest.mark.parametrize("w,h", [(1001, 631), (797, 803)])
+@pytest.mark.parametrize("dtype,skip,keyhole", [("i16", 1, False), ("i16", 0, True), ("f32", 1, True),
+                                                ("f32", 0, False), ("u8", 1, False)])
+def test_two_samples_in_flight_march_as_one(gpu_ctx, w, h, dtype, skip, keyhole):
+    """A single view of many long rays gathers two samples at a time, a plan's
+    persistent schedule one: the same samples in the same order, so the same
+    bits.  Noise about the threshold (runs of one and two samples, steps back),
+    a constant block, empty space, rays that end within a pair, a window."""
+    import torch
+    n, spacing = (200, 66, 61), (1.0, 1.1, 1.2)
+    rng = np.random.default_rng(w)
+    z, y, x = np.meshgrid(*[np.linspace(-1, 1, k) for k in n[::-1]], indexing="ij")
+    vol = np.where(x * x + y * y + z * z < 0.7, rng.uniform(-60.0, 100.0, n[::-1]), 0.0)
+    vol[20:40, 20:40, 60:100] = 90.0
+    if dtype == "u8":
+        vol = np.maximum(vol, 0.0)
+    vol = np.rint(vol).astype({"f32": np.float32, "i16": np.int16, "u8": np.uint8}[dtype])
+    c = configs.volume_center(n, spacing)
+    cam = configs.drr_camera(c, 0.5, h, sod=400.0, sid=800.0, fov=300.0, half_extent=125.0)
+    v, _ = abi.posed_view(cam, [0.05, 0.1, -0.08, 1.0, -2.0, 0.5], c, w, h, spacing=spacing, with_derivatives=True)
+    if keyhole:
+        v.n_keyhole_planes = 2
+        v.keyhole_planes[:8] = [1.0, 0.0, 0.0, -85.0, -1.0, 0.0, 0.0, 120.0]
+    march = configs.march_params({"step_scale": 0.4, "term_T": 0.0, "jitter": 1, "skip_rule": skip})
+    drr = configs.drr_params({"intercept": -1e-4, "slope": 1e-4, "offset": 1.0, "output": abi.DRR_F32_L,
+                              "ref_termination": 0})
+    vh = H.gpu_volume(gpu_ctx, vol, spacing)
+    plan = abi.DrrPlan(gpu_ctx, vh, [v], march, drr)
+    plan.set_schedule(abi.SCHED_PERSISTENT)
+    one = torch.full((plan.total,), float("nan"), device="cuda")
+    two = torch.full((h, w), float("nan"), device="cuda")
+    plan.render(one)
+    abi.render_drr(gpu_ctx, vh, v, march, drr, two)
+    torch.cuda.synchronize()
+    a, b = one.cpu().numpy(), two.cpu().numpy().ravel()
+    assert a.max() > 0.05 and (a == 0.0).any()
+    np.testing.assert_array_equal(a, b)
+    plan.close()
+    vh.close()
+
+
 @pytest.mark.parametrize("name,n,size,cam", [
     ("rays along x", (40, 24, 33), (37, 21), dict(d=(1.0, 0.0, 0.0), dist=400.0, fov=16.0)),
     ("down z, wide pixels", (30, 45, 26), (9, 14), dict(d=(0.05, 0.02, -1.0), dist=300.0, fov=20.0)),
