@@ -37,7 +37,7 @@ HBM_PEAK_GBS = 8000.0
 # wave64 VALU instructions per second: 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles
 VALU_PEAK_GINST = 256 * 4 * 2.4 / 4
 COUNTERS = ROOT / "profiles" / "kernel_counters.json"
-DRR_KERNEL = "drr_kernel<Cells<HalfPair,0,true>,true,true,false,false>"
+DRR_KERNEL = "drr_ahead_kernel<Cells<HalfPair,0,true>,true,false>"
 
 
 def log(msg: str) -> None:
