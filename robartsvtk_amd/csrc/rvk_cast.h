@@ -1,5 +1,7 @@
 // rvk_cast.h -- arguments of the compositing casters.
 #pragma once
+#include <cmath>
+
 #include "rvk_internal.h"
 #include "rvk_march.h"
 
@@ -118,6 +120,38 @@ inline void set_ranges(DrrMarchArgs& m, const rvk_volume* vol, int frame) {
 inline bool quad_ok(const rvk_view* v, const rvk_march_params* m) {
   return m->precise && m->term_T <= 1.0f && v->n_keyhole_planes == 0;
 }
+
+// Whether four lanes per ray pay.  A quad forms its ray four times over
+// (about 0.055 ns a ray on the device) and takes samples in chunks of four; it
+// gains on every gather, the more the further apart a one-lane wave's rays
+// are.  So one lane wins where pixels are many per voxel column (rho) and
+// rays composite few samples: at most k, ln(term) over ln(1 - the smallest
+// opacity of the table).  Measured over 64^3 to 512^3 volumes, 256^2 to
+// 3840x2160 views and opacities of 0.02 to 1 (one lane / four, us): tables of
+// opacity 1, 128^3 at 1400x1100 (rho 94) 1D 135 / 263, unshaded 122 / 217, 2D
+// 148 / 233, with gradient magnitude 135 / 190, dual 160 / 276, in/ex
+// 164 / 302; 256^3 at 1280x1024 (rho 20, k 12) 1D 256 / 350, 2D 308 / 350;
+// opacity 0.1 (k 39) at rho 94 1D 402 / 454, 2D 434 / 415; but ramps (k
+// without bound) 128^3 at rho 94 1D 566 / 427, 2D 1670 / 1243, and 400^3 of
+// opacity 1 at rho 10 524 / 476: the larger the cells beside the 256 MiB
+// cache, the later.  At rho above 3.5 samples per ray (64^3 at 1400x1100) the
+// set-up alone decides: 1D 252 / 258, gradient magnitude 216 / 259.  The
+// unshaded 1D sample is the cheapest: for it also at above 40 N^2 rays of N
+// samples (ramps, 64^3 of 64 samples at 400^2 31 / 36, 128^3 of 128 at 1024x768
+// 102 / 121, of 256 176 / 159).  `share` is k / rho at the crossing, by caster.
+inline bool quad_pays(const rvk_volume* v, const rvk_view* view, float step_len, float least, float term, float share,
+                      bool unshaded = false) {
+  const double rays = (double)view->width * view->height;
+  const double bytes = 8.0 * (double)dtype_size(v->dtype) * (double)v->n_cells;
+  const double rho = rays / std::pow((double)v->dims[0] * v->dims[1] * v->dims[2], 2.0 / 3.0);
+  if (rays < 100000.0) return true;
+  const double n = longest_ray(v, step_len);
+  if (rho >= 3.5 * n || (unshaded && rays >= 40.0 * n * n)) return false;
+  if (rho < 12.0 * std::max(1.0, bytes / (double)(256 << 20))) return true;
+  const double k = least >= 1.0f ? 1.0 : term > 0.0f ? std::log((double)term) / std::log1p(-(double)least) : 1e30;
+  return k > share * rho;
+}
+constexpr float kQuadShare1d = 1.5f, kQuadShareUnshaded = 8.0f, kQuadShareGradmag = 1.5f, kQuadShareGradient = 0.5f;
 
 constexpr int kQuadDealLog2 = 4;  // workgroups of 8x8 pixels in runs of a 32x32 square
 

@@ -453,7 +453,9 @@ int rvk_render_1d(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk_tf1d
                       !std::isfinite(tf->p.gradient_multiplier));
   const bool skip = march->skip_rule != 0, pr = march->precise != 0;
   set_ranges(a.m, vol, frame);
-  if (quad_ok(view, march)) return launch_quad_1d(a, vol, frame, skip, grad, lds, nblk, ctx->stream);
+  if (quad_ok(view, march) && quad_pays(vol, view, a.step_len, tf->least, march->term_T,
+                                        grad ? kQuadShare1d : kQuadShareUnshaded, !grad))
+    return launch_quad_1d(a, vol, frame, skip, grad, lds, nblk, ctx->stream);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
 #define RVK_L1D(S, G, P) \
@@ -513,7 +515,9 @@ int rvk_render_2d(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk_tf2d
   const bool skip = march->skip_rule != 0, dual = tf->kcells != nullptr, gm = use_gradmag != 0;
   const bool pr = march->precise != 0;
   // without keyhole planes no sample takes the keyhole TF
-  if (quad_ok(view, march)) return launch_quad_2d(a, vol, frame, skip, gm, lds, nblk, ctx->stream);
+  if (quad_ok(view, march) && quad_pays(vol, view, a.step_len, tf->least, march->term_T,
+                                        gm ? kQuadShareGradmag : kQuadShareGradient))
+    return launch_quad_2d(a, vol, frame, skip, gm, lds, nblk, ctx->stream);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
 #define RVK_L2D(S, D, G)                                                                              \

@@ -297,7 +297,9 @@ int rvk_render_2d_inex(rvk_ctx* ctx, const rvk_volume* vol, int frame, const rvk
   const bool skip = march->skip_rule != 0, pr = march->precise != 0;
   set_ranges(a.m, vol, frame);
   // (its keyhole window is a test, not a jump)
-  if (pr && march->term_T <= 1.0f) return launch_quad_inex(a, vol, frame, skip, lds, nblk, ctx->stream);
+  if (pr && march->term_T <= 1.0f &&
+      quad_pays(vol, view, a.step_len, tf->inex_least, march->term_T, kQuadShareGradient))
+    return launch_quad_inex(a, vol, frame, skip, lds, nblk, ctx->stream);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
 #define RVK_LIE(S, P) hipLaunchKernelGGL((inex_kernel<CV, S, P>), dim3(nblk), dim3(256), lds, ctx->stream, a)
@@ -356,7 +358,8 @@ int rvk_render_dual(rvk_ctx* ctx, const rvk_volume* vol1, const rvk_volume* vol2
   if (!rc) rc = frame_drop_half(vol2, frame, ctx->stream);
   if (rc) return rc;
   set_ranges(a.m, vol1, frame);
-  if (quad_ok(view, march)) return launch_quad_dual(a, vol1, vol2, frame, skip, lds, nblk, ctx->stream);
+  if (quad_ok(view, march) && quad_pays(vol1, view, a.step_len, tf->least, march->term_T, kQuadShareGradient))
+    return launch_quad_dual(a, vol1, vol2, frame, skip, lds, nblk, ctx->stream);
   return dispatch_frame<false>(vol1, frame, [&](auto tag1) {
     using CV = decltype(tag1);
     return dispatch_frame<false>(vol2, frame, [&](auto tag2) {

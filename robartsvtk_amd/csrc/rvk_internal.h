@@ -53,6 +53,7 @@ struct rvk_tf1d {
   rvk_ctx* ctx = nullptr;
   int n = 0;
   float* tables = nullptr;  // device: alpha[n], galpha[n], r[n], g[n], b[n]
+  float least = 1.0f;       // smallest positive alpha, times that of galpha
   rvk_tf1d_params p{};
 };
 
@@ -92,6 +93,8 @@ struct rvk_tf2d {
   uint32_t* inex_occ = nullptr;
   uint32_t* inex_col = nullptr;  // column bitmap of flag bit 0 (col_words)
   std::vector<float> alpha_host;  // the opacity table, kept for the flags
+  float least = 1.0f;       // smallest positive alpha
+  float inex_least = 1.0f;  // smallest alpha of the cells with flag bit 0
 };
 
 // Largest 2D TF whose opacity bitmap the caster stages in LDS (8 KiB; 16 KiB
@@ -173,6 +176,14 @@ inline int check_march(const rvk_march_params* m) {
   if (!(m->step_scale > 0.0f) || !(m->step_scale < __builtin_huge_valf()))
     return fail(RVK_ERR_INVALID_ARGUMENT, "step_scale must be positive and finite");
   return RVK_OK;
+}
+
+// Smallest positive value of a table (1 if it has none).
+inline float least_positive(const float* v, size_t n) {
+  float m = __builtin_huge_valf();
+  for (size_t i = 0; i < n; ++i)
+    if (v[i] > 0.0f && v[i] < m) m = v[i];
+  return m < __builtin_huge_valf() ? m : 1.0f;
 }
 
 // Samples along the longest axis of the volume.

@@ -20,9 +20,9 @@
 // 2D with gradient magnitude 512^3 u16 1920x1080 4555 -> 2872 (another scene
 // 2549 -> 2068, at 3840x2160 8250 -> 6448), with gradients per sample
 // 11636 -> 5353; shaded 2D 301x257x180 1280x720 1134 -> 871; in/ex 256x256x200
-// 640x480 626 -> 281; dual 320x320x211 1024x768 1225 -> 516.  There is no size
-// measured at which the one-lane casters are faster, so they are left to the
-// views these do not march (quad_ok).
+// 640x480 626 -> 281; dual 320x320x211 1024x768 1225 -> 516.  The one-lane
+// casters take the views that these do not march (quad_ok) and those of many
+// rays with few samples each (quad_pays).
 #pragma once
 #include "rvk_cast.h"
 

@@ -970,6 +970,7 @@ int rvk_tf1d_create(rvk_ctx* ctx, int n, const float* alpha, const float* galpha
   t->ctx = ctx;
   t->n = n;
   t->p = *p;
+  t->least = least_positive(alpha, n) * (std::isfinite(p->gradient_multiplier) ? least_positive(&h[n], n) : 1.0f);
   hipError_t e = hipMalloc((void**)&t->tables, h.size() * sizeof(float));
   if (e != hipSuccess) { delete t; return hip_fail(e, "hipMalloc(tf1d)"); }
   e = hipMemcpy(t->tables, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice);
@@ -1093,6 +1094,7 @@ int rvk_tf2d_create(rvk_ctx* ctx, int n, const float* const tables[8], const flo
     return rc;
   }
   t->alpha_host.assign(tables[0], tables[0] + (size_t)n * n);
+  t->least = least_positive(tables[0], (size_t)n * n);
   *out = t;
   return RVK_OK;
 }
@@ -1112,6 +1114,10 @@ int rvk_tf2d_set_inex(rvk_tf2d* t, const float* inex) {
   std::vector<uint8_t> flags(nn);
   for (size_t c = 0; c < nn; ++c)
     flags[c] = (uint8_t)(((inex[c] > 0.0f || t->alpha_host[c] > 0.0f) ? 1u : 0u) | (inex[c] > 0.5f ? 2u : 0u));
+  // a marked cell without opacity composites nothing: no bound on the samples
+  t->inex_least = least_positive(t->alpha_host.data(), nn);
+  for (size_t c = 0; c < nn; ++c)
+    if ((flags[c] & 1u) && !(t->alpha_host[c] > 0.0f)) t->inex_least = 0.0f;
   RVK_HIP(hipMalloc((void**)&t->inex_flags, nn));
   hipError_t e = hipMemcpy(t->inex_flags, flags.data(), nn, hipMemcpyHostToDevice);
   if (e != hipSuccess) {

@@ -1,0 +1,110 @@
+"""Calls whose fastest route depends on their sizes or data: each takes no
+longer than the route it could have had instead, measured in the same process,
+with the same results."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from robartsvtk_amd import abi, configs
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def _us(call) -> float:
+    """Microseconds a call: the best of seven runs of about 3 ms each."""
+    import torch
+    call()
+    torch.cuda.synchronize()
+    e0, e1 = torch.cuda.Event(True), torch.cuda.Event(True)
+    best, n = float("inf"), 4
+    for _ in range(8):
+        e0.record()
+        for _ in range(n):
+            call()
+        e1.record()
+        torch.cuda.synchronize()
+        us = e0.elapsed_time(e1) * 1000.0 / n
+        n = int(min(60, max(4, 3000.0 / us)))
+        best = min(best, us)
+    return best
+
+
+def _body(n, seed=0, noise=0.0):
+    """int16 CT of an ellipsoid in air; noise: standard deviation of the air's."""
+    rng = np.random.default_rng(seed)
+    z, y, x = np.meshgrid(*[np.linspace(-1, 1, n, dtype=np.float32)] * 3, indexing="ij")
+    inside = (x / 0.8) ** 2 + (y / 0.6) ** 2 + (z / 0.85) ** 2 < 1.0
+    tissue = rng.standard_normal(x.shape, dtype=np.float32) * 20.0 + 40.0
+    air = rng.standard_normal(x.shape, dtype=np.float32) * noise - 1000.0
+    return np.rint(np.where(inside, tissue, air)).astype(np.int16)
+
+
+def _view(n, extent, W, h, sod=2.0):
+    """A view that a volume of `extent` mm a side about fills."""
+    sp = (extent / n,) * 3
+    c = configs.volume_center((n, n, n), sp)
+    d = np.array([1.0, 0.4, 0.3]) / np.linalg.norm([1.0, 0.4, 0.3])
+    cam = abi.camera(c + sod * extent * d, c, (0, 0, 1), 30.0, (0.9 * extent, 3.1 * extent))
+    return sp, abi.compute_view(cam, W, h, spacing=sp)
+
+
+def _empty_window(view):
+    """A keyhole plane that leaves every ray outside: the window is empty, but
+    the view takes the casters that march one lane per ray."""
+    v = abi.View.from_buffer_copy(view)
+    v.n_keyhole_planes = 1
+    v.keyhole_planes[:4] = [1.0, 0.0, 0.0, -1e6]
+    return v
+
+
+# A ray of an opaque table ends at its first sample: four lanes per ray took
+# 1.4 to 2.0 times one lane's time here.
+@pytest.mark.parametrize("caster", ["1d", "1d unshaded", "2d", "2d gradient magnitude", "dual", "inex"])
+def test_opaque_tables_on_magnified_volumes_take_one_lane_per_ray(gpu_ctx, caster):
+    import torch
+    n, W, h, m = 128, 1400, 1100, 256
+    sp, view = _view(n, 256.0, W, h)
+    vol = _body(n)
+    vh, vh2 = H.gpu_volume(gpu_ctx, vol, sp), H.gpu_volume(gpu_ctx, vol[::-1].copy(), sp)
+    lo, w = -1024.0, 2500.0
+    alpha = (np.arange(m) >= 0.4 * m).astype(np.float32)
+    rgb = np.random.default_rng(1).uniform(0, 1, (m, 3)).astype(np.float32)
+    out = torch.empty((h, W, 4), dtype=torch.uint8, device="cuda")
+    full = np.ones((m, m), np.float32)
+    tab = {"alpha": full * alpha, "red": 0.9 * full, "green": 0.5 * full, "blue": 0.2 * full, "ambient": 0.4 * full,
+           "diffuse": 0.6 * full, "specular": 0.2 * full, "specular_power": 12.0 * full}
+    march, over = (configs.march_params({"step_scale": 1.0, "term_T": t, "jitter": 1, "skip_rule": 1})
+                   for t in (1.0 / 64.0, 1.0000001))
+    if caster.startswith("1d"):
+        p = (abi.Tf1dParams(lo, 1 / w, 0.0, float("inf"), 1.0, 0.0, 0.0, 1.0) if caster.endswith("unshaded") else
+             abi.Tf1dParams(lo, 1 / w, 0.0, 1 / w, 0.4, 0.6, 0.2, 10.0))
+        tf = abi.TF1D(gpu_ctx, alpha, rgb, p, galpha=full[0])
+        call = lambda v, mp: abi.render_1d(gpu_ctx, vh, tf, v, mp, out)
+    else:
+        tf = abi.TF2D(gpu_ctx, tab, configs.tf2d_params(configs.tf2d_params_for(lo, lo + w, 0.0, 512.0)))
+        if caster == "dual":
+            dp = abi.DualParams(lo, 1 / w, lo, 1 / w)
+            call = lambda v, mp: abi.render_dual(gpu_ctx, vh, vh2, tf, dp, v, mp, out)
+        elif caster == "inex":
+            tf.set_inex(0.3 * full * alpha)
+            call = lambda v, mp: abi.render_2d_inex(gpu_ctx, vh, tf, v, mp, out, False)
+        else:
+            gm = caster.endswith("magnitude")
+            if gm:
+                vh.compute_gradmag(0, 512.0)
+            call = lambda v, mp: abi.render_2d(gpu_ctx, vh, tf, v, mp, out, gm)
+    # the in/ex caster takes one lane for thresholds above 1, the others for a
+    # view with keyhole planes
+    one = (view, over) if caster == "inex" else (_empty_window(view), march)
+    us, ref_us = _us(lambda: call(view, march)), _us(lambda: call(*one))
+    call(view, march)
+    got = out.clone()
+    if caster != "inex":
+        call(*one)
+        assert torch.equal(got, out)
+    assert int((got[..., 3] > 0).sum()) > W * h // 10
+    for o in (tf, vh, vh2):
+        o.close()
+    assert us <= 1.2 * ref_us, (us, ref_us)
