@@ -7,19 +7,23 @@ namespace rvk {
 // A 16x16-pixel tile per workgroup, the tiles (of a super-tile of 4x4) dealt
 // to the XCDs in runs of 8: the march passes over runs of empty and constant
 // bricks, so a band of tiles per XCD would leave the XCDs of the bands
-// through air idle (256^3 CT at 1024^2 387 us, 1400^2 698 us; deals of 1, 2,
-// 4, 8, 16 and 32 tiles 375 / 365 / 361 / 360 / 382 / 488 us at 1024^2).
+// through air idle (256^3 CT of 512-sample rays, us, in bands / dealt in runs of
+// 1, 2, 4, 8, 16 and 32 tiles: at 1024^2 260 / 240 / 240 / 232 / 231 / 235 / 307,
+// at 1400^2 472 / 372 / 368 / 366 / 364 / 364 / 362; 400^3 at 1024^2
+// 669 / 556 / 553 / 554 / 568 / 596 / 822).
 //
 // Half of a launch's waves end at once in air, and the long rays of the rest
-// make little more than one round of the 8192 the device holds, 3.9 waves per
-// SIMD on average with the VALU 59 % busy: the second sample in flight fills
-// that.  One sample at a time against two (us, int16 CT): 256^3 of 512-sample
-// rays at 1024^2 319 / 290 and 386 / 355 (two scenes), without the skip rule
-// 402 / 376, at 1400x1100 350 / 327, 400^3 at 900^2 461 / 389, 360^3 at
-// 1400x1100 529 / 480; 256-sample rays at 900x800 169 / 155.  Rays of 128
-// samples (128^3 at 1024^2) 107 / 112: they are left to drr_kernel.
+// make little more than one round of the 8192 the device holds: the second
+// sample in flight fills the wait for the first.  Registers for 8 waves per
+// SIMD (7 without the bound: 390 / 363 us at 1400^2).  drr_kernel against
+// this, us, for three bodies -- CT in clean air, in air with noise (values that
+// contribute or not at random), tissue filling the volume: 256^3 at 560^2
+// 261 / 131, 392 / 348, 256 / 182; at 1024^2 453 / 232, 553 / 604, 451 / 444; at
+// 1400^2 833 / 364, 869 / 861, 831 / 735; at 2048^2 1531 / 696, 1588 / 1657,
+// 1547 / 1468; 400^3 at 1024^2 1684 / 568, 2069 / 2046, 1149 / 881.  Without the
+// skip rule 256^3 at 1024^2 437 / 217, 434 / 418, 438 / 402.
 template <typename CV, bool SKIP, bool KEY>
-__global__ __launch_bounds__(256) void drr_ahead_kernel(DrrArgs a) {
+__global__ __launch_bounds__(256, 8) void drr_ahead_kernel(DrrArgs a) {
   int x, y;
   tile_pixel(xcd_deal(blockIdx.x, kDealLog2), a.tiles_x, x, y);
   if (x >= a.v.W || y >= a.v.H) return;

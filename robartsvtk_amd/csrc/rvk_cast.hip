@@ -21,9 +21,8 @@ namespace rvk {
 
 // KEY = false: the view has no keyhole planes; TERM = false: no termination
 // (the accumulated sum is never compared).  For the marches that neither
-// drr_lanes_kernel nor drr_ahead_kernel takes: many short rays without
-// termination, which pass over runs, the reference's positions and
-// termination.
+// drr_lanes_kernel nor drr_ahead_kernel takes: many short rays, the
+// reference's positions and termination.
 template <typename CV, bool SKIP, bool PRECISE, bool KEY, bool TERM>
 __global__ __launch_bounds__(256) void drr_kernel(DrrArgs a) {
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
@@ -31,8 +30,7 @@ __global__ __launch_bounds__(256) void drr_kernel(DrrArgs a) {
   tile_pixel(tile, a.tiles_x, x, y);
   if (x >= a.v.W || y >= a.v.H) return;
   const Ray r = form_ray(a.g, a.v, a.step_len, x, y);
-  const float v = drr_march<CV, SKIP, PRECISE, false, PRECISE && !TERM, KEY, TERM>(cells_of<CV>(a.vol), a.g, a.m, r,
-                                                                                  x, y);
+  const float v = drr_march<CV, SKIP, PRECISE, false, false, KEY, TERM>(cells_of<CV>(a.vol), a.g, a.m, r, x, y);
   drr_store(a, x, y, v);
 }
 

@@ -13,20 +13,28 @@ struct DrrSchedule {
 };
 
 // One view of `rays` rays.  The device holds 8192 waves, and 64 rays are one
-// wave: below about 600 thousand rays it waits on chains of dependent
-// samples, which more lanes per ray shorten; the chunks' bookkeeping costs
-// throughput above.  Measured (us, skip rule, int16 CT, 1 / 2 / 4 / 8 / 16
-// lanes): 256^3 of 512-sample rays at 64^2 261 / 157 / 80 / 43 / 24, 128^2
-// 265 / 159 / 83 / 48 / 38, 360^2 208 / 137 / 91 / -, 512^2 262 / 191 / 180 / -,
-// 724^2 236 / 254 / 274, 1024^2 360 / 426 / 480; 400^3 724^2 368 / 316 / 358;
-// 128^3 of 128-sample rays at 128^2 64 / 40 / 23 / 15 / 12, 360^2 60 / 44 / 41 / 43,
-// 512^2 53 / 63 / 59.  Short rays have no runs worth finding (128^3 at 200^2
-// 24 us without, 36 with) and share their cells within an XCD's band, and so
-// does the smallest launch (256^3 at 64^2: 24 us without runs, 29 with).
+// wave: below that it waits on chains of dependent samples, which more lanes
+// per ray shorten; the chunks' bookkeeping costs throughput above.  Measured
+// with the skip rule on int16 CT, us.  1 / 2 / 4 / 8 / 16 lanes, 256^3 of
+// 512-sample rays at 64^2 261 / 157 / 80 / 43 / 24, 128^2 265 / 159 / 83 / 48 / 38;
+// 128^3 of 128-sample rays at 128^2 64 / 40 / 23 / 15 / 12.  Four lanes against
+// drr_ahead_kernel's one, bodies in clean air / tissue throughout: 512-sample
+// rays at 400^2 120 / 168 and 137 / 156, 480^2 147 / 268 and 142 / 177, 560^2
+// 189 / 309 and 130 / 180; 256-sample rays at 300^2 54 / 76 and 85 / 98, 400^2
+// 82 / 93 and 86 / 89; 800-sample rays at 520^2 311 / 521 and 338 / 803, 700^2
+// 472 / 830 and 489 / 828: the longer the rays, the later they cross.
+// Short rays have no runs worth finding (128^3 at 200^2 24 us without, 36 with)
+// and share their cells within an XCD's band, and so does the smallest launch
+// (256^3 at 64^2: 24 us without runs, 29 with); many of them are drr_kernel's
+// (drr_kernel / drr_ahead_kernel in clean air and with noise, 128-sample rays
+// at 430^2 56 / 41 and 59 / 60, 460^2 54 / 47 and 57 / 65, 64-sample rays at
+// 460^2 20 / 24 and 22 / 29, 1024^2 56 / 59 and 59 / 73).
 inline DrrSchedule drr_schedule(const rvk_volume* vol, long long rays, float step_len) {
   if (rays <= 24576) return {4, false, false};
-  if (longest_ray(vol, step_len) >= 192.0f) return {rays <= 300000 ? 2 : rays <= 600000 ? 1 : 0, true, true};
-  return rays <= 200000 ? DrrSchedule{2, false, false} : DrrSchedule{0, false, true};
+  const float n = longest_ray(vol, step_len);
+  if (n >= 192.0f) return {rays <= std::max(150000.0f, 400.0f * n) ? 2 : 0, true, true};
+  if (rays <= 100000) return {2, false, false};
+  return {0, n >= 96.0f && rays <= 200000, true};
 }
 
 // log2 of the lanes per ray for a plan's forward of `rays` rays in all (in its
