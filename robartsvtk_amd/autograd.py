@@ -12,13 +12,12 @@ the differentiable inputs.
     loss.backward()                            # poses.grad from the HIP adjoint
 
 The forward is rvk_drr_plan_render and the backward rvk_drr_plan_backward
-(pose adjoint and, when the volume requires grad, the brick-driven volume
-adjoint).  The plan holds one set of views and one volume frame; every forward
-records which poses and volume it rendered, and its backward loads them back
-into the plan when another forward has replaced them since (several renders in
-one loss, line searches).  Nothing here computes on the CPU except the
-per-view camera matrices and their pose derivatives (rvk_posed_view, double
-precision).
+(pose adjoint and, when the volume requires grad, the volume adjoint).  The
+plan holds one set of views and one volume frame; every forward records which
+poses and volume it rendered, and its backward loads them back into the plan
+when another forward has replaced them since (several renders in one loss,
+line searches).  Nothing here computes on the CPU except the per-view camera
+matrices and their pose derivatives (rvk_posed_view, double precision).
 """
 from __future__ import annotations
 

@@ -9,6 +9,7 @@ namespace rvk {
 struct BatchView {
   ViewGeom v;
   float dm[96];      // d(view_to_voxels)/d pose_i, i = 0..5 (baked, row major)
+  float inv[16];     // inverse of view_to_voxels: voxel position -> (vx, vy, z, 1) * w
   long long pix_off; // first pixel of this view in the packed image buffer
   int tiles16_x;
   int pad;

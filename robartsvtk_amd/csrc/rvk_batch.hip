@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -326,6 +327,7 @@ __global__ __launch_bounds__(64) void pose_views_kernel(const PoseGeom* __restri
   BatchView& b = views[v];
   for (int k = 0; k < 16; ++k) b.v.m[k] = m[k];
   for (int k = 0; k < 96; ++k) b.dm[k] = dm[k];
+  pose::baked_inverse(m, b.inv);
 }
 
 struct PoseUpdateArgs {
@@ -384,7 +386,10 @@ struct rvk_drr_plan {
   double* d_stats = nullptr;  // n_views x 8
   float* d_pose_part = nullptr;  // n_items x 6
   unsigned long long* d_vg_acc = nullptr;  // per voxel, the volume gradient's sums, allocated by its first call
+  RayRec* d_vg_rays = nullptr;             // or per pixel, its ray records, by the first call that goes by bricks
   unsigned* d_vg_slots = nullptr;          // its largest |coef|
+  double vg_tiles = 0.0;  // 16x16-pixel tiles whose central ray meets the volume
+  double vg_span = 0.0;   // distance in voxels between neighbouring ones, mean across and down
   float* d_jac = nullptr;        // 6 x total pixels, allocated with the plan when it has pose derivatives
   int schedule = RVK_SCHED_GRID;
   int waves_per_simd = 4;
@@ -437,6 +442,8 @@ int fill_views(rvk_drr_plan* p, const rvk_view* views, const float* dview, std::
     std::memset(&b, 0, sizeof(b));
     b.v = view_geom(&views[v]);
     if (dview) std::memcpy(b.dm, dview + 96 * (size_t)v, sizeof(b.dm));
+    // inverse of the baked matrix (Gauss-Jordan, partial pivoting)
+    pose::baked_inverse(views[v].view_to_voxels, b.inv);
     b.tiles16_x = (views[v].width + 15) / 16;
   }
   return RVK_OK;
@@ -454,7 +461,9 @@ static uint32_t morton3(uint32_t x, uint32_t y, uint32_t z) {
   return k;
 }
 
-static void work_orders(const rvk_drr_plan* p, const rvk_view* views, std::vector<int2>& by_view,
+// Also counts the tiles whose central ray meets the volume, and measures how
+// far apart neighbouring ones lie across and down the views (vg_by_tiles).
+static void work_orders(rvk_drr_plan* p, const rvk_view* views, std::vector<int2>& by_view,
                         std::vector<int2>& by_region) {
   by_view.resize(p->n_items);
   for (int v = 0; v < p->n_views; ++v)
@@ -464,7 +473,10 @@ static void work_orders(const rvk_drr_plan* p, const rvk_view* views, std::vecto
   struct Tile { uint32_t key; int v, macro; };
   std::vector<Tile> tiles;
   tiles.reserve(p->n_items / 4);
+  double hit = 0.0, apart[2] = {0.0, 0.0}, pairs[2] = {0.0, 0.0};
+  std::vector<std::array<double, 3>> mid;  // the chords' midpoints (NaN: none), of a view's tiles so far
   for (int v = 0; v < p->n_views; ++v) {
+    mid.clear();
     const rvk_view& vw = views[v];
     const float* m = vw.view_to_voxels;
     const int tx = (vw.width + 15) / 16, n_macro = (p->item_begin[v + 1] - p->item_begin[v]) / 4;
@@ -492,16 +504,30 @@ static void work_orders(const rvk_drr_plan* p, const rvk_view* views, std::vecto
         }
       }
       uint32_t key = 0xffffffffu;
+      mid.push_back({std::nan(""), 0.0, 0.0});
       if (ok && t0 <= t1) {
         const double tm = 0.5 * (t0 + t1);
+        std::array<double, 3>& c = mid.back();
         uint32_t g[3];
-        for (int a = 0; a < 3; ++a)
-          g[a] = (uint32_t)std::min(31.0, std::max(0.0, std::floor((pt[0][a] + tm * (pt[1][a] - pt[0][a])) / cell)));
+        for (int a = 0; a < 3; ++a) {
+          c[a] = pt[0][a] + tm * (pt[1][a] - pt[0][a]);
+          g[a] = (uint32_t)std::min(31.0, std::max(0.0, std::floor(c[a] / cell)));
+        }
         key = morton3(g[0], g[1], g[2]);
+        hit += 1.0;
+        for (int k = 0; k < 2; ++k) {
+          if (k == 0 ? mc % tx == 0 : mc < tx) continue;
+          const std::array<double, 3>& o = mid[mc - (k == 0 ? 1 : tx)];
+          if (std::isnan(o[0])) continue;
+          apart[k] += std::hypot(c[0] - o[0], c[1] - o[1], c[2] - o[2]);
+          pairs[k] += 1.0;
+        }
       }
       tiles.push_back(Tile{key, v, mc});
     }
   }
+  p->vg_tiles = hit;
+  p->vg_span = pairs[0] > 0.0 && pairs[1] > 0.0 ? std::sqrt(apart[0] / pairs[0] * (apart[1] / pairs[1])) : 1e30;
   std::stable_sort(tiles.begin(), tiles.end(), [](const Tile& a, const Tile& b) { return a.key < b.key; });
   by_region.resize(p->n_items);
   size_t i = 0;
@@ -561,6 +587,23 @@ BatchArgs batch_args(const rvk_drr_plan* p, float* out) {
   a.shape = p->shape;
   use_order(p, a, p->order);
   return a;
+}
+
+// Whether the volume adjoint goes by ray tiles (rvk_volgrad.hip) or by voxel
+// bricks (rvk_volbrick.hip): by tiles where these fill the device (6 workgroups
+// on each of 256 CUs; or more of them than half the bricks, which fill it no
+// better) and their rays are close enough for some layers of the box they
+// share in LDS.  Tiles / bricks, us, f32: 16384 tiles 7.7 voxels apart in 256^3
+// 4050 / 7860; 5184 at 15 1494 / 2315; 2704 at 21 1632 / 1375, in 200^3 at 17
+// 850 / 1007; 1225 at 7.7 in 256^3 499 / 536; 625 at 10.7 455 / 398; 169 at 21
+// 614 / 257; 784 at 39 3196 / 655; 64 at 63 1038 / 255; 1296 at 47 in 400^3
+// 10320 / 2056, 2500 at 17 2156 / 2264; 324 at 7.6 in 64^3 82 / 117, 81 at 7.5
+// 75 / 40; 658 at 16 in 400x64x64 494 / 165.
+bool vg_by_tiles(const rvk_drr_plan* p) {
+  const int* n = p->vol->dims;
+  double bricks = 1.0;
+  for (int a = 0; a < 3; ++a) bricks *= (n[a] + kVgEdge - 1) / kVgEdge;
+  return p->vg_span <= 18.0 && p->vg_tiles >= std::min(1000.0, 0.5 * bricks);
 }
 
 // log2 of the lanes per ray of the plan's forward (grad: with Jacobians).  A
@@ -784,6 +827,7 @@ int rvk_drr_plan_destroy(rvk_drr_plan* p) {
   hipFree(p->d_stats);
   hipFree(p->d_pose_part);
   if (p->d_vg_acc) hipFree(p->d_vg_acc);
+  if (p->d_vg_rays) hipFree(p->d_vg_rays);
   if (p->d_vg_slots) hipFree(p->d_vg_slots);
   if (p->d_jac) hipFree(p->d_jac);
   if (p->d_pose_geom) hipFree(p->d_pose_geom);
@@ -1035,7 +1079,6 @@ int rvk_drr_plan_backward(rvk_drr_plan* p, const float* images, const float* dld
   if (grad_pose && !p->d_jac) return fail(RVK_ERR_NOT_READY, "the plan was created without pose derivatives (dview)");
   RVK_HIP(hipSetDevice(p->ctx->device));
   hipStream_t s = p->ctx->stream;
-  const int blocks = (p->n_items + 3) / 4;
   if (grad_pose) {
     AdjArgs aa;
     aa.b = batch_args(p, const_cast<float*>(images));
@@ -1077,16 +1120,27 @@ int rvk_drr_plan_backward(rvk_drr_plan* p, const float* images, const float* dld
       return e;
     };
     const int* d = p->vol->dims;
-    RVK_HIP(need(p->d_vg_acc, sizeof(unsigned long long) * (size_t)d[0] * d[1] * d[2], (void**)&p->d_vg_acc));
     RVK_HIP(need(p->d_vg_slots, sizeof(unsigned) * kVgSlots * kVgSlotStride, (void**)&p->d_vg_slots));
+    bool tiles = vg_by_tiles(p);
+    if (tiles) {
+      const hipError_t e =
+          need(p->d_vg_acc, sizeof(unsigned long long) * (size_t)d[0] * d[1] * d[2], (void**)&p->d_vg_acc);
+      if (e != hipSuccess && e != hipErrorOutOfMemory) return hip_fail(e, "hipMalloc(volume gradient)");
+      if (e != hipSuccess) (void)hipGetLastError();
+      tiles = e == hipSuccess;  // a volume's sums that do not fit: the bricks need only the pixels' rays
+    }
+    if (!tiles)
+      RVK_HIP(need(p->d_vg_rays, sizeof(RayRec) * (size_t)p->pix_off[p->n_views], (void**)&p->d_vg_rays));
     VolGradArgs va;
     va.b = batch_args(p, nullptr);
     va.img = images;
     va.dldi = dldi;
     va.slots = p->d_vg_slots;
     va.acc = p->d_vg_acc;
+    va.rays = p->d_vg_rays;
     va.grad = grad_vol;
-    const int rc = launch_volume_grad(va, p->vol, p->frame, s);
+    const int rc = tiles ? launch_volume_grad(va, p->vol, p->frame, s)
+                         : launch_volume_grad_bricks(va, p->vol, p->frame, s);
     if (rc) return rc;
   }
   return RVK_OK;

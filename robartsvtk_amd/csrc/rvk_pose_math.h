@@ -147,5 +147,14 @@ __host__ __device__ inline bool posed_view(const double pv[16], const double vox
   return true;
 }
 
+// Inverse of a baked float matrix (screen->voxel): voxel position ->
+// (vx, vy, z, 1) * w, as floats; zero if singular.
+__host__ __device__ inline void baked_inverse(const float mb[16], float out[16]) {
+  double m[16], mi[16];
+  for (int k = 0; k < 16; ++k) m[k] = mb[k];
+  const bool ok = invert(m, mi);
+  for (int k = 0; k < 16; ++k) out[k] = ok ? (float)mi[k] : 0.0f;
+}
+
 }  // namespace pose
 }  // namespace rvk

@@ -17,16 +17,14 @@
 // volume's by global atomics.  So each sample is gathered once, in the order
 // of the rays, and passes over empty bricks as the forward does.  Bound by
 // VALU issue (about 95 instructions a sample) and the wait for the gather.
-// (One workgroup per 8^3-voxel brick, re-marching the stretch of every ray
-// that meets it, gathered each sample 1.4 times over and kept 55 % of its
-// lanes: 7858 us and a ray record pass for the 256^3 case below.)
+// A tile whose rays lie far apart has room for few layers or none, and few
+// tiles leave the device idle: such plans go brick by brick (rvk_volbrick.hip).
 #include "rvk_volgrad.h"
 
 #include <type_traits>
 
 namespace rvk {
 
-constexpr int kVgNonFinite = 1 << 30;
 // Sums a workgroup holds (25 KiB: 6 workgroups per CU, as its registers allow)
 // and the most layers of cells in a slab.  Volume gradient, us, with room for
 // 1536 / 2560 / 3200 / 3840 / 5120 sums: 256^3 16 x 512^2 (a tile spans 8 voxels)
@@ -36,88 +34,19 @@ constexpr int kVgNonFinite = 1 << 30;
 constexpr int kVgCap = 3200;
 constexpr int kVgMaxLayers = 8;
 
-struct VgRay {
-  V3<float> p0c, inc;
-  int n;
-  float coef, cs, ci, kw0, kw1;
-};
-
-// The ray of a pixel with the forward's samples, opacities and keyhole window.
-__device__ __forceinline__ VgRay vg_ray(const VolGradArgs& a, const BatchView& bv, int x, int y) {
-  const VolGeom& g = a.b.g;
-  const Ray r = form_ray(g, bv.v, a.b.step_len, x, y);
-  const float j = ray_offset(a.b.m.jitter, x, y);
-  const long long pi = bv.pix_off + (long long)y * bv.v.W + x;
-  const float I = a.img[pi];
-  const float dLdI = a.dldi[pi];
-  const float ds = ray_length(g, r.inc);
-  VgRay q;
-  q.p0c = V3<float>{(r.start.x + j * r.inc.x) + 0.5f, (r.start.y + j * r.inc.y) + 0.5f,
-                    (r.start.z + j * r.inc.z) + 0.5f};
-  q.inc = r.inc;
-  q.n = step_count(r.num_steps - j);
-  // the rays the precise forward march takes no samples of (drr_march)
-  if (!samples_in_cells(g, q.p0c, q.inc, q.n)) q.n = 0;
-  const int es = q.n - (int)ceilf(r.exclude_start), ee = q.n - (int)floorf(r.exclude_end);
-  q.kw0 = (float)(q.n - es);
-  q.kw1 = (float)(q.n - ee);
-  q.ci = a.b.m.intercept * -ds;
-  q.cs = a.b.m.slope * -ds;
-  // d loss / d mu at a sample = (d loss / d L) * ds * slope, with dL/dI = -I for exp(-L)
-  const float dLdL = (a.b.m.output == RVK_DRR_F32_EXP_NEG_L) ? -dLdI * I : dLdI;
-  q.coef = dLdL * ds * a.b.m.slope;
-  return q;
-}
-
-// The pixel of a thread in workgroup blk's tile: four 8x8 items.
-__device__ __forceinline__ const BatchView& vg_pixel(const VolGradArgs& a, int blk, int& x, int& y) {
-  const int2 vt = a.b.work[blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
-  const BatchView& bv = a.b.views[__builtin_amdgcn_readfirstlane(vt.x)];
-  const int local = __builtin_amdgcn_readfirstlane(vt.y), macro = local >> 2, q = local & 3;
-  const int lane = (int)(threadIdx.x & 63u);
-  x = (macro % bv.tiles16_x) * 16 + (q & 1) * 8 + (lane & 7);
-  y = (macro / bv.tiles16_x) * 16 + (q >> 1) * 8 + (lane >> 3);
-  return bv;
-}
-
 __global__ __launch_bounds__(256) void vg_clear_kernel(VolGradArgs a, long long n) {
   const long long i = (long long)blockIdx.x * 512 + threadIdx.x;
   if (i < n) a.acc[i] = 0ull;
   if (i + 256 < n) a.acc[i + 256] = 0ull;
-  if (blockIdx.x == 0 && threadIdx.x < kVgSlots) a.slots[threadIdx.x * kVgSlotStride] = 0u;
+  if (blockIdx.x == 0) vg_clear_slots(a);
 }
 
-// The largest |coef| of a tile's rays with samples, into one of the slots.
 __global__ __launch_bounds__(256) void vg_coef_kernel(VolGradArgs a) {
-  __shared__ float s_m[4];
   int x, y;
   const BatchView& bv = vg_pixel(a, blockIdx.x, x, y);
   float m = 0.0f;
-  if (x < bv.v.W && y < bv.v.H) {
-    const VgRay q = vg_ray(a, bv, x, y);
-    // rays without samples add nothing; a non-finite coefficient poisons the call
-    if (q.n > 0) m = isfinite(q.coef) ? fabsf(q.coef) : __builtin_huge_valf();
-  }
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0)
-    atomicMax(a.slots + (blockIdx.x % kVgSlots) * kVgSlotStride,
-              __float_as_uint(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]))));
-}
-
-// k = 30 - e for the largest |coef| = f 2^e (f in [0.5, 1)): every scaled
-// contribution |coef w 2^k| (w <= 1) is below 2^30 and rounds into an int32.
-__device__ __forceinline__ int vg_scale(const unsigned* slots) {
-  float m = __uint_as_float(slots[(threadIdx.x & 63) * kVgSlotStride]);
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  int e = 0;
-  if (m > 0.0f) frexpf(m, &e);
-  return __builtin_amdgcn_readfirstlane(isfinite(m) ? 30 - e : kVgNonFinite);
-}
-
-__device__ __forceinline__ unsigned long long vg_fixed(float v) {
-  return (unsigned long long)(long long)(int)__builtin_rintf(v);
+  if (x < bv.v.W && y < bv.v.H) m = vg_magnitude(vg_ray(a, bv, x, y));
+  vg_collect(a, m);
 }
 
 // The 8 corner contributions of the sample at q, corner voxel (i - 1 + dx,
@@ -369,7 +298,6 @@ __global__ __launch_bounds__(256, 6) void vg_scatter_kernel(VolGradArgs a) {
 // voxels [8b - 1, 8b + 8], so a brick whose voxels there are all <= 0 stays 0.
 // (A voxel is read as the trilinear value at its own cell corner, weights
 // exactly 0, which is its value in every cell encoding.)
-constexpr int kVgEdge = 8;
 template <typename CV>
 __global__ __launch_bounds__(256) void vg_finish_kernel(VolGradArgs a) {
   const VolGeom& g = a.b.g;

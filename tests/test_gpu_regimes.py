@@ -137,3 +137,111 @@ def test_single_views_without_runs_cost_the_plain_march(gpu_ctx, n, W, step, noi
     assert torch.equal(images[0], images[1])
     assert float(images[0].min()) < 0.9
     assert us[0] <= 1.25 * us[1], us
+
+
+# ---------------------------------------------------------------------------
+# The volume gradient by ray tiles and by voxel bricks
+def _grad_plan(ctx, vh, sp, n, views, output=abi.DRR_F32_L):
+    march = configs.march_params({"step_scale": 0.6, "term_T": 0.0, "jitter": 1, "skip_rule": 0})
+    drr = configs.drr_params({"intercept": 0.0, "slope": 1.0, "offset": 1.0, "output": output, "ref_termination": 0})
+    return abi.DrrPlan(ctx, vh, views, march, drr)
+
+
+def _orbit_view(n, sp, d, w, h, fov=40.0, dist=2.2):
+    ext = max(k * s for k, s in zip(n, sp))
+    c, d = configs.volume_center(n, sp), np.asarray(d, float) / np.linalg.norm(d)
+    cam = abi.camera(c + dist * ext * d, c, (0, 0, 1) if abs(d[2]) < 0.9 else (0, 1, 0), fov / 1.4,
+                     (0.5 * ext, (dist + 2.0) * ext))
+    return abi.compute_view(cam, w, h, spacing=sp)
+
+
+@pytest.mark.parametrize("d", [(1, 0.1, 0.05), (-1, 0.05, 0.1), (0.1, 1, 0.1), (0.05, -1, -0.1), (0.05, 0.02, 1),
+                               (0.1, 0.1, -1), (0.7, -0.6, -0.5)])
+@pytest.mark.parametrize("dtype,keyhole", [("f32", False), ("f32", True), ("i16", False)])
+def test_volume_gradient_is_the_same_by_tiles_and_by_bricks(gpu_ctx, d, dtype, keyhole):
+    """Copies of a view whose d loss / d image is zero add nothing, but make
+    the tiles enough for the route by tiles (1248 against 0.5 * 1248 bricks);
+    alone the view goes by bricks.  Rays along every axis in both senses."""
+    import torch
+    n, sp = (92, 60, 97), (1.0, 1.3, 0.9)
+    rng = np.random.default_rng(5)
+    vol = np.maximum(rng.uniform(-0.02, 0.04, n[::-1]), 0.0).astype(np.float32)
+    vol[:, :20] = 0.0
+    if dtype == "i16":
+        vol = np.rint(vol * 1e4).astype(np.int16)
+    view = _orbit_view(n, sp, d, 150, 131)
+    if keyhole:
+        view.n_keyhole_planes = 2
+        view.keyhole_planes[:8] = [1.0, 0.2, 0.0, -0.3 * n[0], -1.0, 0.0, 0.1, 0.6 * n[0]]
+    vh = H.gpu_volume(gpu_ctx, vol, sp)
+    grads = []
+    for copies in (1, 24):
+        plan = _grad_plan(gpu_ctx, vh, sp, n, [view] * copies)
+        img = torch.zeros(plan.total, device="cuda")
+        plan.render(img)
+        dldi = torch.zeros(plan.total, device="cuda")
+        dldi[: plan.offsets[1]] = torch.from_numpy(np.random.default_rng(6).uniform(-1, 1, plan.offsets[1])).cuda()
+        g = torch.full((vol.size,), float("nan"), device="cuda")
+        plan.backward(img, dldi, grad_volume=g)
+        torch.cuda.synchronize()
+        grads.append(g)
+        plan.close()
+    vh.close()
+    assert torch.equal(grads[0], grads[1])
+    assert int((grads[0] != 0).sum()) > vol.size // 20
+
+
+# One 64x64 view took 1674 us by tiles, a 256x256 one 622.
+@pytest.mark.parametrize("n,views", [(256, 1), (128, 4)])
+def test_volume_gradient_of_fewer_rays_costs_no_more(gpu_ctx, n, views):
+    import torch
+    sp = (256.0 / n,) * 3
+    vol = np.maximum(1.0 + _body(n) / 1000.0, 0.0).astype(np.float32) * 0.02
+    vh = H.gpu_volume(gpu_ctx, vol, sp)
+    g = torch.empty(vol.size, device="cuda")
+    us = []
+    for w in (64, n):
+        plan = _grad_plan(gpu_ctx, vh, sp, (n,) * 3,
+                          [_orbit_view((n,) * 3, sp, (np.cos(0.7 * i), np.sin(0.7 * i), 0.2), w, w)
+                           for i in range(views)])
+        img, dldi = torch.zeros(plan.total, device="cuda"), torch.ones(plan.total, device="cuda")
+        plan.render(img)
+        us.append(_us(lambda: plan.backward(img, dldi, grad_volume=g)))
+        plan.close()
+    vh.close()
+    assert us[0] <= 1.1 * us[1], us
+
+
+def test_volume_gradient_where_its_sums_do_not_fit(gpu_ctx):
+    """8 bytes a voxel for the sums of the route by tiles are not to be had:
+    the gradient goes by bricks, with the same bits."""
+    import torch
+    n, sp = (1024, 1024, 640), (0.25, 0.25, 0.4)
+    vol = torch.randint(0, 3, (n[2], n[1], n[0]), device="cuda", dtype=torch.uint8,
+                        generator=torch.Generator(device="cuda").manual_seed(1))
+    vol[:, 300:] = 0
+    vh = abi.Volume(gpu_ctx, n, sp, np.uint8)
+    vh.set_frame(0, vol)
+    del vol
+    view = _orbit_view(n, sp, (0.2, 1.0, 0.3), 1000, 900)
+    got, hog = [torch.full((n[0] * n[1] * n[2],), float("nan"), device="cuda") for _ in range(2)], None
+    for i in range(2):
+        plan = _grad_plan(gpu_ctx, vh, sp, n, [view])
+        img, dldi = torch.zeros(plan.total, device="cuda"), torch.ones(plan.total, device="cuda")
+        plan.render(img)
+        if i == 1:
+            torch.cuda.synchronize()
+            torch.cuda.empty_cache()
+            free = torch.cuda.mem_get_info()[0]
+            assert free > 8 * n[0] * n[1] * n[2]
+            hog = torch.empty(free - (3 << 30), dtype=torch.uint8, device="cuda")
+        plan.backward(img, dldi, grad_volume=got[i])
+        torch.cuda.synchronize()
+        plan.close()
+    del hog
+    vh.close()
+    same = torch.equal(got[0], got[1])
+    live = int((got[0] != 0).sum())
+    del got
+    torch.cuda.empty_cache()
+    assert same and live > n[0] * n[1] * n[2] // 100
