@@ -302,7 +302,14 @@ int rvk_post_shade_inex(rvk_ctx* ctx, int width, int height, const rvk_shade_par
  *                         other XCDs' queues until all are empty.
  * rvk_drr_plan_autotune times the candidates on this plan and keeps the
  * fastest; rvk_drr_plan_capture records the launch sequence in a hipGraph
- * that rvk_drr_plan_render then replays. */
+ * that rvk_drr_plan_render then replays.
+ *
+ * A plan's results do not depend on its schedule, tile shape or work order.
+ * The precise march without termination puts 1 to 16 lanes on a ray by the
+ * plan's total of rays; the lanes' partial sums (f64 for L, f32 for the pose
+ * Jacobian) are added in their own order, so a view's L can differ by an ulp,
+ * and its registration gradient by a few 1e-6 of the largest entry, between
+ * plans of different totals and from rvk_render_drr. */
 typedef struct rvk_drr_plan rvk_drr_plan;
 
 typedef enum rvk_schedule { RVK_SCHED_GRID = 1, RVK_SCHED_PERSISTENT = 2 } rvk_schedule;

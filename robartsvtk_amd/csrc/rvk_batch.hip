@@ -618,16 +618,18 @@ int launch_forward(rvk_drr_plan* p, float* out, hipStream_t s, bool jac = false)
   a.shape = jac ? p->jac_shape : p->shape;
   use_order(p, a, jac ? p->jac_order : p->order);
   const bool skip = p->march.skip_rule != 0, pr = p->march.precise != 0;
-  // several lanes per ray are part of the default schedule and tile
-  if ((pr || jac) && a.shape == RVK_TILE_8X8 && (jac ? p->jac_schedule : p->schedule) == RVK_SCHED_GRID)
-    if (const int ls = plan_lanes(p, jac)) return launch_batch_lanes(a, p->vol, p->frame, skip, jac, ls, s);
+  const bool persistent = (jac ? p->jac_schedule : p->schedule) == RVK_SCHED_PERSISTENT;
+  const long long groups = (long long)p->n_cu * (jac ? p->jac_waves_per_simd : p->waves_per_simd);
+  if (persistent) hipLaunchKernelGGL(reset_queues_kernel, dim3(1), dim3(64), 0, s, p->d_queues);
+  if (pr || jac)
+    if (const int ls = plan_lanes(p, jac)) {
+      const long long n = (((long long)p->n_items << ls) + 3) / 4;
+      return launch_batch_lanes(a, p->vol, p->frame, skip, jac, ls, persistent ? (unsigned)std::min(groups, n) : 0u, s);
+    }
   return dispatch_frame(p->vol, p->frame, [&](auto tag) {
     using CV = decltype(tag);
-    const int sched = jac ? p->jac_schedule : p->schedule;
-    const int wps = jac ? p->jac_waves_per_simd : p->waves_per_simd;
-    if (sched == RVK_SCHED_PERSISTENT) {
-      hipLaunchKernelGGL(reset_queues_kernel, dim3(1), dim3(64), 0, s, p->d_queues);
-      const int blocks = std::max(1, std::min(p->n_cu * wps, (p->n_items + 3) / 4));
+    if (persistent) {
+      const unsigned blocks = (unsigned)std::min(groups, ((long long)p->n_items + 3) / 4);
 #define RVK_LP(S, P, J)                                                                                     \
   do {                                                                                                      \
     if (p->drr.ref_termination)                                                                             \

@@ -37,9 +37,11 @@ inline DrrSchedule drr_schedule(const rvk_volume* vol, long long rays, float ste
   return {0, n >= 96.0f && rays <= 200000, true};
 }
 
-// log2 of the lanes per ray for a plan's forward of `rays` rays in all (in its
-// grid schedule), always with runs.  grad: the march also sums gradients, and every lane forms the ray's set-up and shares its tangents,
-// so more lanes pay less.  Measured (us, register on f32 / int16 volumes,
+// log2 of the lanes per ray for a plan's forward of `rays` rays in all, always
+// with runs; the plan's alone, so that its results do not depend on its tuned
+// schedule, tile and order (the lanes set the order of a ray's sums).  grad: the
+// march also sums gradients, and every lane forms the ray's set-up and shares
+// its tangents, so more lanes pay less.  Measured (us, register on f32 / int16 volumes,
 // 1 / 2 / 4 / 8 / 16 lanes): 200^3 1 x 128^2 133 / 78 / 51 / 40 / 39, 2 x 128^2
 // 139 / 82 / 57 / 53 / 63, 2 x 200^2 151 / 92 / 74 / 77 / 84, 8 x 200^2
 // 266 / 198 / 195 / 218, 4 x 400^2 211 / 213 / 260, 8 x 400^2 325 / 357; 256^3 (512
@@ -57,8 +59,9 @@ inline int batch_lanes(const rvk_volume* vol, long long rays, float step_len, bo
 int launch_drr_lanes(const DrrArgs& a, const rvk_volume* vol, int frame, bool skip, int ls, int nblk, hipStream_t s);
 // One view, one lane per ray, tiles dealt (rvk_ahead.hip).
 int launch_drr_ahead(const DrrArgs& a, const rvk_volume* vol, int frame, bool skip, int nblk, hipStream_t s);
-// A plan's forward (jac: with the pose Jacobians).
+// A plan's forward (jac: with the pose Jacobians); persistent: the workgroups
+// of that schedule, whose queues are cleared, or 0.
 int launch_batch_lanes(const BatchArgs& a, const rvk_volume* vol, int frame, bool skip, bool jac, int ls,
-                       hipStream_t s);
+                       unsigned persistent, hipStream_t s);
 
 }  // namespace rvk

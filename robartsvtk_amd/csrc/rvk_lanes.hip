@@ -30,11 +30,19 @@ int launch_drr_lanes(const DrrArgs& a, const rvk_volume* vol, int frame, bool sk
   });
 }
 
-// The wave's part of an 8x8-pixel work item.
-__device__ __forceinline__ void item_part_pixel(int tiles16_x, int local, int part, int ls, int& x, int& y) {
-  const int macro = local >> 2;
-  const int lane = (int)(threadIdx.x & 63u);
-  morton_pixel(((local & 3) << 6) | (part << (6 - ls)) | (lane >> ls), x, y);
+// The wave's part of a work item of the plan's tile shape.
+__device__ __forceinline__ void item_part_pixel(int shape, int tiles16_x, int local, int part, int ls, int& x, int& y) {
+  const int macro = local >> 2, q = local & 3;
+  const int p = (part << (6 - ls)) | ((int)(threadIdx.x & 63u) >> ls);  // pixel of the item
+  if (shape == RVK_TILE_16X4) {
+    x = p & 15;
+    y = q * 4 + (p >> 4);
+  } else if (shape == RVK_TILE_4X16) {
+    x = q * 4 + (p & 3);
+    y = p >> 2;
+  } else {
+    morton_pixel((q << 6) | p, x, y);
+  }
   x += (macro % tiles16_x) * 16;
   y += (macro / tiles16_x) * 16;
 }
@@ -47,16 +55,13 @@ __device__ __forceinline__ void group_sum(V3<float>& v, int S) {
   }
 }
 
+// Part w mod 2^ls of work item w >> ls.
 template <typename CV, bool SKIP, bool JAC>
-__global__ __launch_bounds__(256) void batch_lanes_kernel(BatchArgs a, int ls) {
-  const int blk = a.deal ? xcd_deal(blockIdx.x, kDealLog2 + ls) : xcd_remap(blockIdx.x, gridDim.x);
-  const int w = blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int item = w >> ls;
-  if (item >= a.n_items) return;
-  const int2 vt = a.work[item];
+__device__ __forceinline__ void lanes_part(const BatchArgs& a, int w, int ls) {
+  const int2 vt = a.work[w >> ls];
   const BatchView& bv = a.views[__builtin_amdgcn_readfirstlane(vt.x)];
   int x, y;
-  item_part_pixel(bv.tiles16_x, __builtin_amdgcn_readfirstlane(vt.y), w & ((1 << ls) - 1), ls, x, y);
+  item_part_pixel(a.shape, bv.tiles16_x, __builtin_amdgcn_readfirstlane(vt.y), w & ((1 << ls) - 1), ls, x, y);
   if (x >= bv.v.W || y >= bv.v.H) return;
   const Ray r = form_ray(a.g, bv.v, a.step_len, x, y);
   const long long pi = bv.pix_off + (long long)y * bv.v.W + x;
@@ -88,18 +93,45 @@ __global__ __launch_bounds__(256) void batch_lanes_kernel(BatchArgs a, int ls) {
   }
 }
 
+template <typename CV, bool SKIP, bool JAC>
+__global__ __launch_bounds__(256) void batch_lanes_kernel(BatchArgs a, int ls) {
+  const int blk = a.deal ? xcd_deal(blockIdx.x, kDealLog2 + ls) : xcd_remap(blockIdx.x, gridDim.x);
+  const int w = blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((w >> ls) >= a.n_items) return;
+  lanes_part<CV, SKIP, JAC>(a, w, ls);
+}
+
+// The persistent schedule (batch_persistent_kernel), over the items' parts.
+template <typename CV, bool SKIP, bool JAC>
+__global__ __launch_bounds__(256) void batch_lanes_persistent_kernel(BatchArgs a, int ls) {
+  const int home = blockIdx.x % kNumXcd;
+  const long long parts = (long long)a.n_items << ls;
+  for (int r = 0; r < kNumXcd; ++r) {
+    const int c = (home + r) % kNumXcd;
+    const int begin = (int)(parts * c / kNumXcd), end = (int)(parts * (c + 1) / kNumXcd);
+    while (true) {
+      int w = 0;
+      if ((threadIdx.x & 63) == 0) w = (int)atomicAdd(&a.queues[c], 1u);
+      w = begin + __builtin_amdgcn_readfirstlane(w);
+      if (w >= end) break;
+      lanes_part<CV, SKIP, JAC>(a, w, ls);
+    }
+  }
+}
+
 int launch_batch_lanes(const BatchArgs& a, const rvk_volume* vol, int frame, bool skip, bool jac, int ls,
-                       hipStream_t s) {
-  const dim3 grid(batch_grid(a, ls));
+                       unsigned persistent, hipStream_t s) {
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
-    if (jac) {
-      if (skip) hipLaunchKernelGGL((batch_lanes_kernel<CV, true, true>), grid, dim3(256), 0, s, a, ls);
-      else hipLaunchKernelGGL((batch_lanes_kernel<CV, false, true>), grid, dim3(256), 0, s, a, ls);
-    } else {
-      if (skip) hipLaunchKernelGGL((batch_lanes_kernel<CV, true, false>), grid, dim3(256), 0, s, a, ls);
-      else hipLaunchKernelGGL((batch_lanes_kernel<CV, false, false>), grid, dim3(256), 0, s, a, ls);
-    }
+    auto go = [&](auto S, auto J) {
+      constexpr bool kSkip = decltype(S)::value, kJac = decltype(J)::value;
+      if (persistent)
+        hipLaunchKernelGGL((batch_lanes_persistent_kernel<CV, kSkip, kJac>), dim3(persistent), dim3(256), 0, s, a, ls);
+      else
+        hipLaunchKernelGGL((batch_lanes_kernel<CV, kSkip, kJac>), dim3(batch_grid(a, ls)), dim3(256), 0, s, a, ls);
+    };
+    if (jac) skip ? go(std::true_type(), std::true_type()) : go(std::false_type(), std::true_type());
+    else skip ? go(std::true_type(), std::false_type()) : go(std::false_type(), std::false_type());
     RVK_HIP(hipGetLastError());
     return (int)RVK_OK;
   });

@@ -245,3 +245,47 @@ def test_volume_gradient_where_its_sums_do_not_fit(gpu_ctx):
     del got
     torch.cuda.empty_cache()
     assert same and live > n[0] * n[1] * n[2] // 100
+
+
+@pytest.mark.parametrize("skip", [0, 1])
+@pytest.mark.parametrize("n_views,w", [(1, 90), (2, 140), (3, 300), (9, 300)])
+def test_plan_results_do_not_depend_on_schedule_tile_or_order(gpu_ctx, n_views, w, skip):
+    """16, 8, 4 and 2 lanes per ray (views of 8100 to 810000 rays in all):
+    images, losses and the registration gradient to the bit."""
+    import torch
+    n, sp = (60, 52, 47), (1.0, 1.1, 1.2)
+    rng = np.random.default_rng(7)
+    vol = np.maximum(rng.uniform(-0.01, 0.02, n[::-1]), 0.0).astype(np.float32)
+    vol[:, :, :15] = 0.0
+    c = configs.volume_center(n, sp)
+    views, dms = [], []
+    for i in range(n_views):
+        cam = configs.drr_camera(c, 0.4 + 0.9 * i, w, sod=300.0, sid=600.0, fov=200.0, half_extent=75.0)
+        v, dm = abi.posed_view(cam, [0.05 * i, 0.1, -0.08, 1.0, -2.0, 0.5], c, w, w, spacing=sp, with_derivatives=True)
+        views.append(v)
+        dms.append(dm)
+    march = configs.march_params({"step_scale": 0.15, "term_T": 0.0, "jitter": 1, "skip_rule": skip})
+    drr = configs.drr_params({"intercept": 0.0, "slope": 1.0, "offset": 1.0, "output": abi.DRR_F32_EXP_NEG_L,
+                              "ref_termination": 0})
+    vh = H.gpu_volume(gpu_ctx, vol, sp)
+    plan = abi.DrrPlan(gpu_ctx, vh, views, march, drr, dview=np.stack(dms))
+    tgt = torch.from_numpy(rng.uniform(0, 1, plan.total).astype(np.float32)).cuda()
+    ref = None
+    for sched, wps in ((abi.SCHED_GRID, 4), (abi.SCHED_PERSISTENT, 2), (abi.SCHED_PERSISTENT, 8)):
+        for shape in (abi.TILE_8X8, abi.TILE_16X4, abi.TILE_4X16):
+            for order in (abi.ORDER_VIEWS, abi.ORDER_REGIONS):
+                plan.set_schedule(sched, wps)
+                plan.set_tile_shape(shape)
+                plan.set_work_order(order)
+                out, reg = (torch.full((plan.total,), float("nan"), device="cuda") for _ in range(2))
+                loss, grad = torch.empty(n_views, device="cuda"), torch.empty(6 * n_views, device="cuda")
+                plan.render(out)
+                plan.register(reg, tgt, loss, grad)
+                torch.cuda.synchronize()
+                got = [out, reg, loss, grad]
+                if ref is None:
+                    ref = got
+                assert all(torch.equal(a, b) for a, b in zip(ref, got)), (sched, wps, shape, order)
+    assert float(ref[0].min()) < 0.95 and float(ref[3].abs().max()) > 0
+    plan.close()
+    vh.close()
