@@ -399,8 +399,7 @@ struct rvk_drr_plan {
   // tile's central ray crosses (all views' tiles of one region together, so
   // an XCD's L2 serves one region's cells to every view)
   int2* d_work[2] = {nullptr, nullptr};
-  int order = 0, jac_order = 0;
-  bool auto_order = true;  // no order set or tuned yet
+  int order = RVK_ORDER_REGIONS, jac_order = RVK_ORDER_REGIONS;
   // the fused registration forward (pose Jacobians) has its own schedule:
   // its per-wave work differs enough that the best choice can differ
   int jac_schedule = RVK_SCHED_GRID;
@@ -545,8 +544,8 @@ static int upload_work_orders(rvk_drr_plan* p, const rvk_view* views) {
   return RVK_OK;
 }
 
-// The order the marches take the tiles in: the plan's, or until one is set or
-// tuned the region order with its tiles dealt to the XCDs in runs of 8.  The
+// The order the marches take the tiles in: view by view in a band per XCD, or by
+// region (a new plan's) with the tiles dealt to the XCDs in runs of 8.  The
 // regions cluster what the views share, and the deal evens out what the runs
 // leave each XCD to do (us, forward / pose adjoint): 64 poses of a 512x512x400
 // CT 25100 / 35250 view by view in bands, 21310 / 31790 so, 4 poses 2996 / 3443
@@ -554,7 +553,7 @@ static int upload_work_orders(rvk_drr_plan* p, const rvk_view* views) {
 // 1683 / 1809 and 1590 / 1741.  Dealing the view-major order is slower there
 // (2500 / 2800: the XCDs then share no view's cells).
 void use_order(const rvk_drr_plan* p, BatchArgs& a, int order) {
-  const bool regions = p->auto_order || order == RVK_ORDER_REGIONS;
+  const bool regions = order == RVK_ORDER_REGIONS;
   a.work = p->d_work[regions ? 1 : 0];
   a.deal = regions;
 }
@@ -885,7 +884,6 @@ int rvk_drr_plan_autotune(rvk_drr_plan* p, float* out, int reps, float* best_ms)
   reps = std::max(1, std::min(reps, 100));
   RVK_HIP(hipSetDevice(p->ctx->device));
   drop_graph(p);
-  p->auto_order = false;
   // schedule x waves per SIMD x wave tile x work order
   const int cand[][2] = {{RVK_SCHED_GRID, 4}, {RVK_SCHED_PERSISTENT, 2}, {RVK_SCHED_PERSISTENT, 4},
                          {RVK_SCHED_PERSISTENT, 8}};
@@ -984,8 +982,7 @@ int rvk_drr_plan_set_work_order(rvk_drr_plan* p, int order) {
   if (!p) return fail(RVK_ERR_INVALID_ARGUMENT, "plan is NULL");
   if (order != RVK_ORDER_VIEWS && order != RVK_ORDER_REGIONS)
     return fail(RVK_ERR_INVALID_ARGUMENT, "unknown work order %d", order);
-  if (p->auto_order || order != p->order || order != p->jac_order) drop_graph(p);
-  p->auto_order = false;
+  if (order != p->order || order != p->jac_order) drop_graph(p);
   p->order = p->jac_order = order;
   return RVK_OK;
 }
