@@ -28,12 +28,13 @@ struct DrrSchedule {
 // (256^3 at 64^2: 24 us without runs, 29 with); many of them are drr_kernel's
 // (drr_kernel / drr_ahead_kernel in clean air and with noise, 128-sample rays
 // at 430^2 56 / 41 and 59 / 60, 460^2 54 / 47 and 57 / 65, 64-sample rays at
-// 460^2 20 / 24 and 22 / 29, 1024^2 56 / 59 and 59 / 73).
+// 460^2 20 / 24 and 22 / 29, 1024^2 56 / 59 and 59 / 73; drr_kernel / four lanes,
+// 64-sample rays at 200^2 18 / 14 and 20 / 18, 300^2 18 / 19 and 20 / 28).
 inline DrrSchedule drr_schedule(const rvk_volume* vol, long long rays, float step_len) {
   if (rays <= 24576) return {4, false, false};
   const float n = longest_ray(vol, step_len);
   if (n >= 192.0f) return {rays <= std::max(150000.0f, 400.0f * n) ? 2 : 0, true, true};
-  if (rays <= 100000) return {2, false, false};
+  if (rays <= (n >= 96.0f ? 100000 : 50000)) return {2, false, false};
   return {0, n >= 96.0f && rays <= 200000, true};
 }
 
@@ -41,12 +42,16 @@ inline DrrSchedule drr_schedule(const rvk_volume* vol, long long rays, float ste
 // with runs; the plan's alone, so that its results do not depend on its tuned
 // schedule, tile and order (the lanes set the order of a ray's sums).  grad: the
 // march also sums gradients, and every lane forms the ray's set-up and shares
-// its tangents, so more lanes pay less.  Measured (us, register on f32 / int16 volumes,
-// 1 / 2 / 4 / 8 / 16 lanes): 200^3 1 x 128^2 133 / 78 / 51 / 40 / 39, 2 x 128^2
-// 139 / 82 / 57 / 53 / 63, 2 x 200^2 151 / 92 / 74 / 77 / 84, 8 x 200^2
-// 266 / 198 / 195 / 218, 4 x 400^2 211 / 213 / 260, 8 x 400^2 325 / 357; 256^3 (512
-// samples) 8 x 200^2 610 / 406 / 362 / 389, 8 x 400^2 793 / 661 / 735, 16 x 512^2
-// 1855 / 1931; its plain render 1590 / 1359 / 1629.
+// its tangents, so more lanes pay less.  Measured (us, register on f32 / int16
+// volumes, 1 / 2 / 4 / 8 / 16 lanes): 200^3 1 x 128^2 133 / 78 / 51 / 40 / 39, 2 x
+// 128^2 139 / 82 / 57 / 53 / 63, 2 x 200^2 151 / 92 / 74 / 77 / 84, 8 x 200^2
+// 266 / 198 / 195 / 218.  Above 400 thousand rays 1 / 2 / 4 lanes, int16 CT in clean
+// air: render 128^3 of 128 samples 4 x 400^2 107 / 100 / 120, with the skip rule
+// 105 / 108 / 128, 16 x 200^2 137 / 116 / 136 and 135 / 126 / 140, 200^3 4 x 400^2
+// 168 / 151 / 197; register 189 / 189 / 228, 180 / 187 / 221, 214 / 208 / 245 and
+// 205 / 205 / 235, 255 / 242 / 313; 256^3 of 512 samples, render
+// 8 x 560^2 761 / 666 / 835 (skip rule 759 / 813 / 973), 40 x 512^2 2818 / 2603 / 3371;
+// register 4 x 560^2 586 / 590 / 725, 6 x 560^2 824 / 883 / 1064.
 inline int batch_lanes(const rvk_volume* vol, long long rays, float step_len, bool grad) {
   if (rays <= 24576) return 4;
   if (rays <= 49152) return 3;

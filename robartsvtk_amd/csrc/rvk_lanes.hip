@@ -8,14 +8,14 @@
 
 namespace rvk {
 
-template <typename CV, bool SKIP>
+template <typename CV, bool SKIP, bool RUNS>
 __global__ __launch_bounds__(256) void drr_lanes_kernel(DrrArgs a, int ls) {
   const int blk = a.deal ? xcd_deal(blockIdx.x, kDealLog2 + ls) : xcd_remap(blockIdx.x, gridDim.x);
   int x, y;
   lanes_pixel(blk, a.tiles_x, ls, x, y);
   if (x >= a.v.W || y >= a.v.H) return;
   const Ray r = form_ray(a.g, a.v, a.step_len, x, y);
-  const float v = drr_march_lanes<CV, SKIP>(cells_of<CV>(a.vol), a.g, a.m, r, x, y, ls);
+  const float v = drr_march_lanes<CV, SKIP, RUNS>(cells_of<CV>(a.vol), a.g, a.m, r, x, y, ls);
   if ((threadIdx.x & ((1 << ls) - 1)) == 0) drr_store(a, x, y, v);
 }
 
@@ -23,8 +23,11 @@ int launch_drr_lanes(const DrrArgs& a, const rvk_volume* vol, int frame, bool sk
   const dim3 grid(a.deal ? deal_grid((long long)nblk << ls, kDealLog2 + ls) : (unsigned)nblk << ls);
   return dispatch_frame(vol, frame, [&](auto tag) {
     using CV = decltype(tag);
-    if (skip) hipLaunchKernelGGL((drr_lanes_kernel<CV, true>), grid, dim3(256), 0, s, a, ls);
-    else hipLaunchKernelGGL((drr_lanes_kernel<CV, false>), grid, dim3(256), 0, s, a, ls);
+    const bool runs = a.m.ranges != nullptr;
+    if (skip && runs) hipLaunchKernelGGL((drr_lanes_kernel<CV, true, true>), grid, dim3(256), 0, s, a, ls);
+    else if (skip) hipLaunchKernelGGL((drr_lanes_kernel<CV, true, false>), grid, dim3(256), 0, s, a, ls);
+    else if (runs) hipLaunchKernelGGL((drr_lanes_kernel<CV, false, true>), grid, dim3(256), 0, s, a, ls);
+    else hipLaunchKernelGGL((drr_lanes_kernel<CV, false, false>), grid, dim3(256), 0, s, a, ls);
     RVK_HIP(hipGetLastError());
     return (int)RVK_OK;
   });
@@ -67,13 +70,13 @@ __device__ __forceinline__ void lanes_part(const BatchArgs& a, int w, int ls) {
   const long long pi = bv.pix_off + (long long)y * bv.v.W + x;
   const bool lead = (threadIdx.x & ((1 << ls) - 1)) == 0;
   if (!JAC) {
-    const float v = drr_march_lanes<CV, SKIP>(cells_of<CV>(a.vol), a.g, a.m, r, x, y, ls);
+    const float v = drr_march_lanes<CV, SKIP, true>(cells_of<CV>(a.vol), a.g, a.m, r, x, y, ls);
     if (lead) a.out[pi] = v;
     return;
   }
   V3<float> A{0, 0, 0}, B{0, 0, 0};
   PoseVisit visit{ray_offset(a.m.jitter, x, y), A, B};
-  const float v = drr_march_lanes<CV, SKIP, true>(cells_of<CV>(a.vol), a.g, a.m, r, x, y, ls, visit);
+  const float v = drr_march_lanes<CV, SKIP, true, true>(cells_of<CV>(a.vol), a.g, a.m, r, x, y, ls, visit);
   if (lead) a.out[pi] = v;
   // the lanes' sums added, lane s forms pose directions s, s + 2^ls, ...
   // (dL/dpose_i = A . dstart_i + B . dinc_i)

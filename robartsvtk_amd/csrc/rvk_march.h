@@ -359,8 +359,8 @@ __device__ __forceinline__ float drr_march(CV vol, const VolGeom& g, const DrrMa
 // in the air at 1024^2, looking always / so: 1012 / 604 us, without the skip rule
 // 793 / 418; in clean air, where the loop without lookups is the shorter,
 // 323 / 232 and 326 / 217; rests of 8 and 16 iterations within 4 %).
-constexpr int kRunRest = 16;   // iterations of drr_march_ahead
-constexpr int kLanesRest = 6;  // chunks of drr_march_lanes
+constexpr int kRunRest = 16;    // iterations of drr_march_ahead
+constexpr int kLanesRest = 24;  // samples of drr_march_lanes, in chunks of a ray's lanes
 
 // The same line integral, the sample after the next gathered along with the
 // next: where the march goes on as it did (sample by sample while samples
@@ -477,7 +477,7 @@ __device__ __forceinline__ float drr_march_ahead(CV vol, const VolGeom& g, const
 // which counts if it contributes, and goes on sample by sample from u).
 // Either way the chunk's first change of run, found in the ballot of the
 // samples' signs, says where the next chunk starts.
-template <typename CV, bool SKIP, bool VG = false, typename F = NoVisit>
+template <typename CV, bool SKIP, bool RUNS, bool VG = false, typename F = NoVisit>
 __device__ __forceinline__ float drr_march_lanes(CV vol, const VolGeom& g, const DrrMarchArgs& a, const Ray& r, int x,
                                                  int y, int ls, F&& visit = F()) {
   const int S = 1 << ls, lane = (int)(threadIdx.x & 63u);
@@ -503,6 +503,7 @@ __device__ __forceinline__ float drr_march_lanes(CV vol, const VolGeom& g, const
   const bool runs = a.ranges != nullptr;
   const RangeWalk w = range_walk(p0c, inc);
   const float flat_lim = fminf(kw0, tend);  // a contributing run ends before the keyhole window
+  const int rest = kLanesRest >> ls;
   if (SKIP) {
     const uint32_t all = (1u << S) - 1u;
     float t = 0.0f;        // the chunk's first sample, the same in the ray's lanes
@@ -542,14 +543,14 @@ __device__ __forceinline__ float drr_march_lanes(CV vol, const VolGeom& g, const
       }
       two = two == whole;
     };
-    if (!runs)
+    if (!RUNS)
       while (t < tend) chunk(false);
     while (t < tend) {
       const float t0 = t;
-      chunk(true);
+      chunk(runs);
       if (__ballot(t - t0 > 2.0f * fS)) continue;  // a run moves a ray on by more than a chunk
 #pragma unroll 1
-      for (int i = 0; i < kLanesRest && t < tend; ++i) chunk(false);
+      for (int i = 0; i < rest && t < tend; ++i) chunk(false);
     }
   } else {
     const float rS = 1.0f / fS;
@@ -571,14 +572,14 @@ __device__ __forceinline__ float drr_march_lanes(CV vol, const VolGeom& g, const
       }
     };
     alpha_prev = __builtin_nanf("");
-    if (!runs)
+    if (!RUNS)
       while (t < tend) take(false);
     while (t < tend) {
       const float t0 = t;
-      take(true);
+      take(runs);
       if (__ballot(t - t0 > fS)) continue;
 #pragma unroll 1
-      for (int i = 0; i < kLanesRest && t < tend; ++i) take(false);
+      for (int i = 0; i < rest && t < tend; ++i) take(false);
     }
   }
   for (int o = 1; o < S; o <<= 1) acc += __shfl_xor(acc, o, 64);
