@@ -153,7 +153,7 @@ inline bool quad_pays(const rvk_volume* v, const rvk_view* view, float step_len,
 }
 constexpr float kQuadShare1d = 1.5f, kQuadShareUnshaded = 8.0f, kQuadShareGradmag = 1.5f, kQuadShareGradient = 0.5f;
 
-constexpr int kQuadDealLog2 = 4;  // workgroups of 8x8 pixels in runs of a 32x32 square
+constexpr int kQuadDealLog2 = 4;  // workgroups of 8x8 pixels in runs of a 64x16 strip
 
 // The same casters with four lanes per ray (rvk_quad.h); nblk is the launch's
 // count of 16x16-pixel tiles.

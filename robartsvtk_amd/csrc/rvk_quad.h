@@ -11,9 +11,10 @@
 // theirs, the chain is a quarter as long, and the ordered compositing of a
 // chunk, by quad broadcasts, costs about 33 VALU instructions per 64 samples
 // of 60 to 250.  Now bound by VALU issue (73 to 95 % busy in the 2D casters).
-// The 16 blocks of a 32x32-pixel square go to one XCD, the squares dealt over
-// the XCDs (runs of 4, 8, 16, 32 and 64 blocks measured within 3 %, a band per
-// XCD 10 to 50 % slower: it leaves the XCDs of the image's rim idle).
+// 16 blocks in a row go to one XCD, which are a strip of 64x16 pixels (four
+// tiles of a super-tile's row), the strips dealt over the XCDs (runs of 4, 8,
+// 16, 32 and 64 blocks measured within 3 %, a band per XCD 10 to 50 % slower: it
+// leaves the XCDs of the image's rim idle).
 //
 // One lane in bands against this, us: 1D 128^3 u8 512^2 108 -> 90, 1024^2
 // 267 -> 249, 128^2 120 -> 57; shaded 1D 250x250x181 int16 800x600 453 -> 282;
