@@ -11,8 +11,10 @@ offset)).
 `roofline` is the resource the DRR kernel comes closest to, VALU issue: its VALU
 instructions per launch (SQ_INSTS_VALU, committed rocprofv3 counter pass,
 profiles/kernel_counters.json) over the live kernel time, against
-256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles per wave64 instruction.  The HBM
-traffic the counters measure and the gather-equivalent bytes (8 voxels per
+256 CUs x 4 SIMDs x 2.4 GHz / the mean issue cycles of a wave64 instruction in
+the kernel's inner loop (recorded beside its counters: plain multiplies, adds
+and moves issue in about 2.3 cycles each, conversions, compares, fractions, mixed
+and 64-bit operations in 4).  The HBM traffic the counters measure and the gather-equivalent bytes (8 voxels per
 sample) are reported beside it.  `cpu_baseline` times the CPU oracle (FP32,
 a -march=native build made on this host, every core of the process's
 affinity) on each configuration and reports every configuration's error
@@ -34,8 +36,8 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 HBM_PEAK_GBS = 8000.0
-# wave64 VALU instructions per second: 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles
-VALU_PEAK_GINST = 256 * 4 * 2.4 / 4
+# VALU issue cycles per ns of the device: 256 CUs x 4 SIMDs x 2.4 GHz
+VALU_GCYCLES = 256 * 4 * 2.4
 COUNTERS = ROOT / "profiles" / "kernel_counters.json"
 DRR_KERNEL = "drr_ahead_kernel<Cells<HalfPair,0,true>,true,false>"
 
@@ -526,12 +528,13 @@ def main() -> int:
     kern_s = r["kernel_ms"] / 1e3
     alg_bytes = r["n_samples"] * 8 * 2 + r["pixels"] * 4
     cnt = kernel_counters(DRR_KERNEL)
-    roof = {"bound": "valu", "unit": "G VALU wave-instructions/s", "peak": VALU_PEAK_GINST,
+    peak = VALU_GCYCLES / (cnt.get("valu_cycles_per_inst", 4.0) if cnt else 4.0)
+    roof = {"bound": "valu", "unit": "G VALU wave-instructions/s", "peak": round(peak, 1),
             "kernel": DRR_KERNEL, "kernel_ms": round(r["kernel_ms"], 4)}
     if cnt:
         ach = cnt["SQ_INSTS_VALU"] / kern_s / 1e9
         hbm = cnt["hbm_bytes"] / kern_s / 1e9
-        roof.update({"achieved": round(ach, 1), "frac": round(ach / VALU_PEAK_GINST, 4), "traffic": cnt["hbm_bytes"],
+        roof.update({"achieved": round(ach, 1), "frac": round(ach / peak, 4), "traffic": cnt["hbm_bytes"],
                      "valu_insts_per_launch": cnt["SQ_INSTS_VALU"], "valu_busy_counters": cnt.get("valu_busy"),
                      "hbm": {"achieved_GBs": round(hbm, 1), "peak": HBM_PEAK_GBS, "frac": round(hbm / HBM_PEAK_GBS, 4)}})
     else:
